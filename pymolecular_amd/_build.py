@@ -34,11 +34,12 @@ FLAGS = [
 ]
 
 
-# per-file flags: the edge-parallel MPNN backward keeps its MFMA accumulators in VGPRs (the VALU reads
+# per-file flags: the edge-parallel kernels keep their MFMA accumulators in VGPRs (the VALU reads
 # every product's result; the AGPR form would copy each one back)
 FILE_FLAGS = {
     "egnn_mpnn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "egnn_eqfwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "egnn_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -198,7 +198,8 @@ int32_t egnn_fwd(const EgnnDims* dims, const EgnnStrides* strides, const void* h
   {
     ProfScope ps(EGNN_K_FWD_EDGE, st);
     const int r = coop_supported(s) ? launch_coop_fwd(s, a, st)
-                  : wide_supported(s) ? launch_wide_fwd(s, a, st) : launch_fwd(s, a, 0, st);
+                  : wide_supported(s) ? launch_wide_fwd(s, a, st)
+                  : f32_split_supported(s) ? launch_f32_fwd(s, a, st) : launch_fwd(s, a, 0, st);
     if ((rc = hip_status(r)) != EGNN_OK) return rc;
   }
   ProfScope ps(EGNN_K_FWD_FIXUP, st);

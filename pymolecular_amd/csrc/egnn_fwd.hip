@@ -383,7 +383,8 @@ static int launch_fwd_t(const FwdArgs& a, int part, hipStream_t st) {
   constexpr int SEGW = O + (EQ ? 4 : 0), SEGP = SEGW + 4;
   const size_t lds = 4 * (size_t)(kTileEdges * SEGP + kTileEdges) * sizeof(float);
   if (part == 0) {
-    if (a.ntiles > 0) {
+    if constexpr (sizeof(T) == 4 && H == 128) return (int)hipErrorInvalidValue;   // egnn_f32.hip
+    else if (a.ntiles > 0) {
       int blocks = (int)std::min<int64_t>(cdiv(a.ntiles, 4), 256 * 2);
       hipLaunchKernelGGL((fwd_edge_kernel<T, H, O, M, NB, EQ>), dim3(blocks), dim3(256), lds, st, a);
     }

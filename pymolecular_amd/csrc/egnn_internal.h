@@ -47,6 +47,12 @@ struct FragSet {
   float* w2mf; // [M]
   float* wdf;  // [H]  w_d in fp32 (EGNN only)
   void* wn;    // [F][2H] activation dtype: [W_n1 | W_n2] side by side (node projections)
+  // fp32, H = 128 (f32_split_supported): the weights in three bf16 parts (egnn_split.h), as 24 KB chunks in the
+  // order the edge kernels use them.  Chunk 2k: rows 32k .. 32k + 31 of the first product's matrix
+  // [row block][k slice][part]; chunk 2k + 1 (EGNN): k slice k of the second's [row block][part].
+  void* s_fwd;   // W_hl^T (and W1_mov^T): pre2, q
+  void* s_bwd;   // W1_mov and W_hl (EGNN), W_hl by k slices alone (MPNN): g_m, g_a1
+  void* s_u;     // W_u [row block][slot slice][part]
 };
 
 struct LayerShape {
@@ -116,6 +122,7 @@ constexpr int64_t kChunkFillEdges = 6144 * 32;
 int64_t factor_chunk_edges(const LayerShape& s);
 size_t fwd_ws_layout(const LayerShape& s, void* base, FwdWs* w);
 size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w);
+size_t fwd_split_extra(const LayerShape& s);   // forward workspace beyond what fp32 weight fragments would take
 // Split-K products [A | 1]^T B over K rows with an M x N result: rows per
 // slice (about 512 blocks of the launcher's tile, slices of 256 rows or more)
 // and the fp32 partial elements that need.  Reductions over kSplitKBig rows or
@@ -292,8 +299,9 @@ int launch_wide_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
 constexpr int kWideBwdBlocks = 256;
 int wide_bwd_blocks(const LayerShape& s);
 int launch_wide_bwd(const LayerShape& s, const BwdArgs& a, int nblk, hipStream_t st);
-// Per-edge geometry records for the cooperative kernels (one thread per edge):
-// forward [E][4] = (delta, r^2); backward [E][8] = (r^2, g_phi, delta, grad x_i / deg).
+// fp32 edge kernels on split operands (egnn_f32.hip): H = O = M = 128
+bool f32_split_supported(const LayerShape& s);
+int launch_f32_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
 int bwd_tile_edges(const LayerShape& s);
 
 // dPQ[n] = [sum_row Gh | sum_csc Gh] (summed in fp32, stored in the activation dtype);

@@ -11,6 +11,7 @@
 // recomputes it per edge).
 #include "egnn_device.h"
 #include "egnn_internal.h"
+#include "egnn_split.h"
 
 namespace egnn {
 
@@ -49,11 +50,29 @@ int make_shape(const EgnnDims* d, LayerShape* s) {
 
 static size_t frag_bytes(int R, int K, size_t esz) { return (size_t)(R / 16) * cdiv(K, 32) * kFragElems * esz; }
 
+// blocks per job of the weight preparation
+static int prep_blocks(const LayerShape& s) {
+  int64_t most = std::max<int64_t>((int64_t)(s.O / 16) * cdiv(s.H, 32) * kFragElems, (int64_t)s.F * 2 * s.H);
+  if (s.eq) most = std::max<int64_t>(most, (int64_t)(s.M / 16) * cdiv(s.O, 32) * kFragElems);
+  most = std::max<int64_t>(most, (int64_t)(s.H / 16) * cdiv(s.KU, 32) * kFragElems);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(most, 256), 1024));
+}
+
 static size_t frag_layout(const LayerShape& s, char* base, FragSet* f, size_t off, bool with_bwd) {
   auto take = [&](size_t bytes) { void* p = base ? base + off : nullptr; off = align_up(off + bytes); return p; };
-  f->hlT = take(frag_bytes(s.O, s.H, s.esz));
-  f->movT = s.eq ? take(frag_bytes(s.M, s.O, s.esz)) : nullptr;
-  f->u = s.NUC ? take(frag_bytes(s.H, s.KU, s.esz)) : nullptr;
+  const bool sp = f32_split_supported(s) && !with_bwd;
+  if (sp) {   // bf16 parts of the weights
+    const size_t one = 3 * frag_bytes(s.O, s.H, 2);
+    f->s_fwd = take(s.eq ? 2 * one : one);
+    f->s_bwd = nullptr;
+    f->s_u = s.NUC ? take(3 * frag_bytes(s.H, s.KU, 2)) : nullptr;
+  } else {
+    f->s_fwd = f->s_bwd = f->s_u = nullptr;
+  }
+  const bool own = !sp;   // the split kernels read their own fragments only
+  f->hlT = own ? take(frag_bytes(s.O, s.H, s.esz)) : nullptr;
+  f->movT = own && s.eq ? take(frag_bytes(s.M, s.O, s.esz)) : nullptr;
+  f->u = own && s.NUC ? take(frag_bytes(s.H, s.KU, s.esz)) : nullptr;
   f->mov = (with_bwd && s.eq) ? take(frag_bytes(s.O, s.M, s.esz)) : nullptr;
   f->hl = with_bwd ? take(frag_bytes(s.H, s.O, s.esz)) : nullptr;
   f->uT = (with_bwd && s.eq) ? take(frag_bytes(16, s.H, s.esz)) : nullptr;
@@ -75,6 +94,12 @@ size_t fwd_ws_layout(const LayerShape& s, void* base, FwdWs* w) {
   w->geo = (float*)(b && geo ? b + off : nullptr);
   if (geo) off = align_up(off + (size_t)std::max<int64_t>(s.E, 1) * 4 * sizeof(float));
   return off;
+}
+
+size_t fwd_split_extra(const LayerShape& s) {
+  if (!f32_split_supported(s)) return 0;
+  const int64_t elems = (int64_t)s.O * s.H + (s.eq ? (int64_t)s.M * s.O : 0) + (int64_t)s.H * s.KU;
+  return (size_t)elems * (3 * 2 - 4);
 }
 
 int64_t splitk_len(int64_t M, int64_t N, int64_t K, bool fold) {
@@ -179,6 +204,9 @@ enum FragKind { FK_WT = 0, FK_W = 1, FK_U = 2, FK_UT = 3 };
 struct FragDesc {
   void* dst; int R, K, nkc, kind, chain;
   const void* src; int64_t ld;
+  // split != 0: the fragments in three bf16 parts each, at fragment (rb / 2) stride + off + ((rb % 2) nkc + kc) 3
+  // (split 1: chunks of two row blocks) or kc stride + off + 3 rb (split 2: chunks of one k slice)
+  int split, stride, off;
 };
 
 // All weight preparation of one layer call in one launch: blockIdx.y selects the
@@ -232,7 +260,14 @@ __device__ void frag_build(const FragDesc& d, int F, int FE, int H, int eq, int 
           break;
       }
     }
-    dst[idx] = from_f32<T>(v);
+    if (sizeof(T) == 4 && d.split) {
+      bf16* p = (bf16*)d.dst + (idx & 511) +
+                (int64_t)kFragElems * (d.split == 1 ? (rb >> 1) * d.stride + d.off + ((rb & 1) * d.nkc + kc) * 3
+                                                    : kc * d.stride + d.off + 3 * rb);
+      split::split1(v, p[0], p[kFragElems], p[2 * kFragElems]);
+    } else {
+      dst[idx] = from_f32<T>(v);
+    }
   }
 }
 
@@ -307,14 +342,22 @@ static int prep_impl(const LayerShape& s, const void* w1, const void* w2, const 
                      hipStream_t st) {
   PrepArgs p{};
   FragDesc* slots[6] = {&p.f0, &p.f1, &p.f2, &p.f3, &p.f4, &p.f5};
-  int64_t most = 0;
   auto add = [&](void* dst, int R, int K, int kind, int chain, const void* src, int64_t ld) {
     if (!dst) return;
-    *slots[p.nfrag++] = FragDesc{dst, R, K, (int)cdiv(K, 32), kind, chain, src, ld};
-    most = std::max<int64_t>(most, (int64_t)(R / 16) * cdiv(K, 32) * kFragElems);
+    *slots[p.nfrag++] = FragDesc{dst, R, K, (int)cdiv(K, 32), kind, chain, src, ld, 0, 0, 0};
+  };
+  auto add3 = [&](void* dst, int R, int K, int kind, int chain, const void* src, int64_t ld, int split, int stride, int off) {
+    if (!dst) return;
+    *slots[p.nfrag++] = FragDesc{dst, R, K, (int)cdiv(K, 32), kind, chain, src, ld, split, stride, off};
   };
   // packed weights: W_hl (H x O), W1mov (O x M); nn.Linear layout: their transposes
   const int kW = s.lin ? FK_W : FK_WT, kWT = s.lin ? FK_WT : FK_W;
+  if (fr.s_fwd) {
+    const int rows = 6 * (s.H / 32), both = rows + (s.eq ? 3 * (s.M / 16) : 0);   // fragments of a chunk, of a chunk pair
+    add3(fr.s_fwd, s.O, s.H, kW, 1, w2, s.lin ? s.H : s.O, 1, both, 0);
+    if (s.eq) add3(fr.s_fwd, s.M, s.O, kW, 1, w1m, s.lin ? s.O : s.M, 2, both, rows);
+    if (s.NUC) add3(fr.s_u, s.H, s.KU, FK_U, 0, w1, s.H, 1, 6 * s.NUC, 0);
+  }
   add(fr.hlT, s.O, s.H, kW, 1, w2, s.lin ? s.H : s.O);                // A[o][h] = W_hl[h][o]
   if (s.eq) add(fr.movT, s.M, s.O, kW, 1, w1m, s.lin ? s.O : s.M);    // A[m][o] = W1mov[o][m]
   if (s.NUC) add(fr.u, s.H, s.KU, FK_U, 0, w1, s.H);
@@ -324,13 +367,12 @@ static int prep_impl(const LayerShape& s, const void* w1, const void* w2, const 
     if (s.eq) add(fr.uT, 16, s.H, FK_UT, 1, w1, s.H);
   }
   p.w1 = w1; p.wn = fr.wn;
-  most = std::max<int64_t>(most, (int64_t)s.F * 2 * s.H);
   p.b2 = b2; p.bx1 = s.eq ? bx1 : nullptr; p.w2m = s.eq ? w2m : nullptr;
   p.wd = s.eq ? w1 : nullptr;
   p.kw = s.lin ? 2 * s.F + (s.eq ? 1 : 0) + s.FE : 0;
   p.b2f = fr.b2f; p.bx1f = fr.bx1f; p.w2mf = fr.w2mf; p.wdf = fr.wdf;
   p.F = s.F; p.FE = s.FE; p.H = s.H; p.O = s.O; p.M = s.M; p.eq = s.eq ? 1 : 0;
-  p.bx = (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(most, 256), 1024));
+  p.bx = prep_blocks(s);
   if (geo && geo->out && geo->E > 0) {
     p.geo = *geo;
     p.geo_blocks = (int)std::min<int64_t>(cdiv(geo->E, 256), 8192);

@@ -1,0 +1,103 @@
+// fp32 products on the bf16 matrix cores (gfx950).
+//
+// v_mfma_f32_16x16x4_f32 runs at 1/16 of the bf16 rate per contracted element, so an fp32 contraction
+// is done as six bf16 products.  A value x is split into three bf16 parts that carry its 24 significand
+// bits exactly: x0 = the upper 16 bits of x (never overflows), x1 = bf16(x - x0), x2 = x - x0 - x1 (both
+// differences are exact, and the last one has at most 8 bits).  a b is then a0 b0 + (a0 b1 + a1 b0) +
+// (a0 b2 + a1 b1 + a2 b0); what is left out, a1 b2 + a2 b1 + a2 b2, is below 2^-23 |a b| at worst and
+// about 2^-27 |a b| rms, of either sign, against the 2^-25 rms of one fp32 rounding.  The bf16 products
+// are exact in fp32.  The large term has an accumulator of its own (K / 32 roundings instead of the K / 4 or
+// more of the fp32 instruction); the five correction terms, 2^-8 of it or less, go to a second one.
+//
+// An infinite operand has no such parts (inf - inf), so the products it enters are NaN where the fp32
+// instruction may give an infinity; a finite one never becomes infinite (x0 is truncated), and a column of
+// the result that no such operand enters is not touched.
+#pragma once
+#include "egnn_device.h"
+
+namespace egnn {
+namespace split {
+
+// a chunk (8 values per lane) in three bf16 parts
+struct Chunk3 { bf16x8 p0, p1, p2; };
+
+__device__ __forceinline__ uint32_t fbits(float x) { return __builtin_bit_cast(uint32_t, x); }
+__device__ __forceinline__ float bitsf(uint32_t u) { return __builtin_bit_cast(float, u); }
+
+// parts of one value (weights, prepared once per call)
+__device__ __forceinline__ void split1(float x, bf16& a, bf16& b, bf16& c) {
+  const float x0 = bitsf(fbits(x) & 0xffff0000u);
+  const float r = x - x0;
+  a = (bf16)x0;
+  b = (bf16)r;
+  c = (bf16)(r - (float)b);
+}
+
+typedef __bf16 bf16x2_ __attribute__((ext_vector_type(2)));
+// the upper halves of two values as one register, x in the low half
+__device__ __forceinline__ uint32_t hi_pair(float x, float y) { return __builtin_amdgcn_perm(fbits(y), fbits(x), 0x07060302u); }
+
+__device__ __forceinline__ Chunk3 split_chunk(const f32x4& lo, const f32x4& hi) {
+  u32x4 q0, q1, q2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x = i < 2 ? lo[2 * i] : hi[2 * i - 4], y = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
+    q0[i] = hi_pair(x, y);
+    const float rx = x - bitsf(fbits(x) & 0xffff0000u), ry = y - bitsf(fbits(y) & 0xffff0000u);
+    bf16x2_ b;
+    b[0] = (bf16)rx;
+    b[1] = (bf16)ry;
+    q1[i] = __builtin_bit_cast(uint32_t, b);
+    bf16x2_ c;
+    c[0] = (bf16)(rx - bitsf(q1[i] << 16));
+    c[1] = (bf16)(ry - bitsf(q1[i] & 0xffff0000u));
+    q2[i] = __builtin_bit_cast(uint32_t, c);
+  }
+  return Chunk3{__builtin_bit_cast(bf16x8, q0), __builtin_bit_cast(bf16x8, q1), __builtin_bit_cast(bf16x8, q2)};
+}
+
+// the six products of one 32-deep slice: hi += a0 b0, lo += the corrections (smallest first)
+__device__ __forceinline__ void mma3(f32x4& hi, f32x4& lo, const Chunk3& a, const Chunk3& b) {
+  mma(lo, a.p2, b.p0);
+  mma(hi, a.p0, b.p0);
+  mma(lo, a.p0, b.p2);
+  mma(lo, a.p1, b.p1);
+  mma(lo, a.p1, b.p0);
+  mma(lo, a.p0, b.p1);
+}
+// the same for two row blocks, their products in turn (no product waits for the one just issued)
+__device__ __forceinline__ void mma3x2(f32x4* hi, f32x4* lo, const Chunk3& a, const Chunk3& d, const Chunk3& b) {
+  mma(lo[0], a.p2, b.p0);
+  mma(lo[1], d.p2, b.p0);
+  mma(hi[0], a.p0, b.p0);
+  mma(hi[1], d.p0, b.p0);
+  mma(lo[0], a.p0, b.p2);
+  mma(lo[1], d.p0, b.p2);
+  mma(lo[0], a.p1, b.p1);
+  mma(lo[1], d.p1, b.p1);
+  mma(lo[0], a.p1, b.p0);
+  mma(lo[1], d.p1, b.p0);
+  mma(lo[0], a.p0, b.p1);
+  mma(lo[1], d.p0, b.p1);
+}
+
+// SiLU of the fp32 path: e^-x as 2^t (1 + d ln 2) with t = fl(-x log2 e) and d its rounding error (the
+// product's by fma, and log2 e's own), so the exponential keeps the accuracy of v_exp_f32 (1 ulp) for every x.
+// x is clamped in the exponent only, where the sigmoid is 0 or 1 to fp32 precision: an infinite x then gives
+// no inf - inf in d (SiLU(inf) = inf, SiLU(-inf) = -inf * 0 = NaN as with expf).
+__device__ __forceinline__ float sigmoid_f32(float x) {
+  const float u = __builtin_amdgcn_fmed3f(x, -120.0f, 120.0f);
+  const float t = u * -1.44269502e+0f;                                   // fl(log2 e)
+  const float d = __builtin_fmaf(u, -1.92596303e-8f, __builtin_fmaf(u, -1.44269502e+0f, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  return __builtin_amdgcn_rcpf(1.0f + e * __builtin_fmaf(d, 0.693147182f, 1.0f));   // e may be inf: a product, no fma
+}
+__device__ __forceinline__ float silu_f32(float x) { return x * sigmoid_f32(x); }
+__device__ __forceinline__ YD silu_yd_f32(float x) {
+  const float s = sigmoid_f32(x);
+  const float y = x * s;
+  return YD{y, __builtin_fmaf(y, 1.0f - s, s)};
+}
+
+}  // namespace split
+}  // namespace egnn

@@ -23,7 +23,10 @@ namespace {
 constexpr size_t kScratchBytes = EGNN_FWD_STATIC_SCRATCH_BYTES;
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// A graph is accepted by the workspace it needs with the weights as fp32 fragments; their three bf16 parts
+// (egnn_split.h) take half as much again, at most kSplitExtra, kept beyond the documented size.
+constexpr size_t kSplitExtra = size_t(1) << 20;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kSplitExtra];
 
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
@@ -59,9 +62,10 @@ extern "C" int32_t egnn_fwd_static(const EgnnDims* dims, const EgnnStrides* stri
   int32_t rc = egnn::make_shape(dims, &s);
   if (rc != EGNN_OK) return rc;
   egnn::FwdWs w;
-  if (egnn::fwd_ws_layout(s, nullptr, &w) > kScratchBytes) return EGNN_ERR_SCRATCH;
+  const size_t extra = egnn::fwd_split_extra(s);
+  if (extra > kSplitExtra || egnn::fwd_ws_layout(s, nullptr, &w) > kScratchBytes + extra) return EGNN_ERR_SCRATCH;
   void* ws = nullptr;
   if ((rc = device_scratch((hipStream_t)stream, &ws)) != EGNN_OK) return rc;
   return egnn_fwd(dims, strides, h, coord, edge_feat, rowptr, col, edge_ids, w1_msg, w2_msg, w1_mov, w2_mov, b1,
-                  b2, bx1, out_msg, out_mov, node_proj, sched, ws, kScratchBytes, stream);
+                  b2, bx1, out_msg, out_mov, node_proj, sched, ws, kScratchBytes + extra, stream);
 }

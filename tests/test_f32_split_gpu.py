@@ -1,0 +1,86 @@
+"""fp32 kernels on split bf16 operands (H = 128) at the edges of their tiles, against the float64 oracle.
+
+Bound: an fp32 product summed over K = 128 terms in any order differs from the exact sum by at most
+128 * 2^-24 = 7.6e-6 of the sum of the terms' magnitudes; normwise (largest difference over largest
+value) 1e-5 therefore holds for any correct fp32 implementation of the layer, as in test_fused_gpu.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import egnn_oracle as orc
+from tests.cases import Case, random_csr
+from tests.test_fused_gpu import check_case, run_fused
+
+pytestmark = pytest.mark.gpu
+
+
+def _degrees(kind):
+    """Rows that end, begin and go on at every 16-edge half and 32-edge tile boundary."""
+    if kind == "one":
+        return [1]
+    if kind == "15":
+        return [15, 0]
+    if kind == "16":
+        return [16]
+    if kind == "17":          # a row over the half boundary, last tile half empty
+        return [3, 0, 14]
+    if kind == "32":
+        return [16, 16]
+    if kind == "33":
+        return [10, 20, 3]
+    if kind == "ones":        # 32 ranks per tile
+        return [1] * 70
+    if kind == "halves":      # ends exactly at halves and tiles, and just beside them
+        return [15, 2, 15, 16, 16, 31, 1, 32, 17, 0, 47, 33, 48, 5]
+    return [200, 0, 3, 100, 31, 65, 7]
+
+
+@pytest.mark.parametrize("eq", [True, False])
+@pytest.mark.parametrize("kind", ["one", "15", "16", "17", "32", "33", "ones", "halves", "long"])
+def test_tile_edges(kind, eq):
+    degs = _degrees(kind) + [0] * 5   # sources besides the row itself (a self edge has no coordinate gradient)
+    rowptr, col = random_csr(len(degs), degs, seed=len(degs))
+    check_case(Case(rowptr, col, 128, 0, 128, 128, 128, seed=31, eq=eq, mean_agg=eq), "fp32")
+
+
+@pytest.mark.parametrize("eq,fe", [(True, 8), (True, 24), (True, 32), (True, 40), (False, 8), (False, 32), (False, 64)])
+def test_edge_feature_slots(eq, fe):
+    """Edge-feature widths around the 32-slot slices (the r^2 slot in the last slice, or alone in one)."""
+    degs = _degrees("halves")
+    rowptr, col = random_csr(len(degs), degs, seed=3)
+    perm = np.random.Generator(np.random.PCG64(3)).permutation(len(col))
+    check_case(Case(rowptr, col, 32, fe, 128, 128, 128, seed=32, eq=eq, edge_ids=perm), "fp32")
+
+
+@pytest.mark.parametrize("eq", [True, False])
+def test_not_finite_rows_stay_apart(eq):
+    """A node with infinite and NaN features makes its own and its neighbours' rows not finite, no others."""
+    degs = np.array([4, 9, 33, 0, 16, 20, 2, 40])
+    rowptr, col = random_csr(len(degs), degs, seed=4)
+    case = Case(rowptr, col, 128, 0, 128, 128, 128, seed=33, eq=eq)
+    ref, _ = case.forward_ref(False)
+    case.h[5, 3], case.h[5, 7] = np.inf, np.nan
+    rows = np.repeat(np.arange(len(degs)), degs)
+    hit = np.unique(np.concatenate([rows[col == 5], rows[rows == 5]]))
+    out = run_fused(case, "fp32", backward=False)["out_msg"]
+    clean = np.setdiff1d(np.arange(len(degs)), hit)
+    assert len(clean) and not np.isfinite(out[hit]).any()
+    assert orc.normwise_rel_err(out[clean], ref[clean]) <= 1e-5
+
+
+def test_extreme_magnitudes():
+    """Features from 1e-30 to the largest finite value: the parts of a split value never overflow."""
+    degs = np.array([5, 30, 3, 8])
+    rowptr, col = random_csr(len(degs), degs, seed=5)
+    case = Case(rowptr, col, 16, 0, 128, 128, 128, seed=34, eq=False)
+    case.h[0] *= 1e-30
+    case.h[1] *= 1e15
+    for k in ("w1_msg", "w2_msg"):
+        case.p[k] = np.abs(case.p[k])
+    case.h = np.abs(case.h).astype(np.float32)
+    check_case(case, "fp32", backward=False)
+    case.h[2] = np.finfo(np.float32).max
+    case.p["w1_msg"] = (case.p["w1_msg"] * 2.0 ** -9).astype(np.float32)
+    check_case(case, "fp32", backward=False)
+    torch.cuda.synchronize()
