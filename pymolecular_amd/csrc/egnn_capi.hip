@@ -345,6 +345,7 @@ int32_t egnn_bwd(const EgnnDims* dims, const EgnnStrides* strides, const void* h
     // chunk_gh (fp32) also the products over the chunk's Gh and its node sums, added to the earlier
     // chunks' (so Gh, Gx and r^2 hold one chunk as well)
     const int TW = bwd_tile_edges(s);
+    const bool sp = f32_split_supported(s);
     const int64_t Lw = (int64_t)(s.H + 1) * s.O, Lm = (int64_t)(s.O + 1) * s.M;
     const int64_t Lwe = (int64_t)s.H * std::max(s.FE, 1);
     const int nc = w.nchunk;
@@ -360,32 +361,45 @@ int32_t egnn_bwd(const EgnnDims* dims, const EgnnStrides* strides, const void* h
       a.tile0 = e0 / TW; a.ntiles = cdiv(e1, TW); a.fbase = e0; a.gbase = gb;
       {
         ProfScope ps(EGNN_K_BWD_EDGE, st);
-        if ((rc = hip_status(launch_bwd(s, a, st))) != EGNN_OK) return rc;
+        if ((rc = hip_status(sp ? launch_f32_bwd(s, a, st) : launch_bwd(s, a, st))) != EGNN_OK) return rc;
       }
-      Gemm2Args g{};
-      g.M = s.H + 1; g.N = s.O; g.K = e1 - e0;
-      g.A = w.Dm1; g.lda = s.H; g.a_bf16 = s.bf16; g.a_kc = 0; g.a_ones_row = s.H;
-      g.B = w.Dga2; g.ldb = s.O; g.b_bf16 = s.bf16; g.b_nc = 1;
-      if ((rc = splitk2(g, one ? w.dWhl : res_w + ch * Lw)) != EGNN_OK) return rc;
-      if (s.eq) {
-        Gemm2Args m{};
-        m.M = s.O + 1; m.N = s.M; m.K = e1 - e0;
-        m.A = w.Dm; m.lda = s.O; m.a_bf16 = s.bf16; m.a_kc = 0; m.a_ones_row = s.O;
-        m.B = w.Dgq; m.ldb = s.M; m.b_bf16 = s.bf16; m.b_nc = 1;
-        if ((rc = splitk2(m, one ? w.dW1m : res_m + ch * Lm)) != EGNN_OK) return rc;
-        Gemm2Args p{};   // dw2_mov = sum_e p[e] g_phi[e]  (g_phi in column 3 of Gx)
-        p.M = s.M; p.N = 1; p.K = e1 - e0;
-        p.A = w.Dp; p.lda = s.M; p.a_bf16 = s.bf16; p.a_kc = 0; p.a_ones_row = -1;
-        p.B = w.Gx + 4 * (e0 - gb) + 3; p.ldb = 4; p.b_bf16 = 0; p.b_nc = 1;
-        if ((rc = splitk2(p, one ? w.dw2m : res_p + ch * s.M)) != EGNN_OK) return rc;
+      if (sp) {   // both factor products in one launch, added to the earlier chunks' partial rows
+        const AtbF32Args p{(const float*)w.Dm1, (const float*)w.Dga2, (const float*)w.Dm, (const float*)w.Dgq,
+                           e1 - e0, atb_f32_len(w.chunkE), w.atb, w.atb_ld, ch > 0};
+        ProfScope ps(EGNN_K_EDGE_WGRAD, st);
+        if ((rc = hip_status(launch_atb_f32(p, s.eq ? 2 : 1, st))) != EGNN_OK) return rc;
+      } else {
+        Gemm2Args g{};
+        g.M = s.H + 1; g.N = s.O; g.K = e1 - e0;
+        g.A = w.Dm1; g.lda = s.H; g.a_bf16 = s.bf16; g.a_kc = 0; g.a_ones_row = s.H;
+        g.B = w.Dga2; g.ldb = s.O; g.b_bf16 = s.bf16; g.b_nc = 1;
+        if ((rc = splitk2(g, one ? w.dWhl : res_w + ch * Lw)) != EGNN_OK) return rc;
+        if (s.eq) {
+          Gemm2Args m{};
+          m.M = s.O + 1; m.N = s.M; m.K = e1 - e0;
+          m.A = w.Dm; m.lda = s.O; m.a_bf16 = s.bf16; m.a_kc = 0; m.a_ones_row = s.O;
+          m.B = w.Dgq; m.ldb = s.M; m.b_bf16 = s.bf16; m.b_nc = 1;
+          if ((rc = splitk2(m, one ? w.dW1m : res_m + ch * Lm)) != EGNN_OK) return rc;
+          Gemm2Args p{};   // dw2_mov = sum_e p[e] g_phi[e]  (g_phi in column 3 of Gx)
+          p.M = s.M; p.N = 1; p.K = e1 - e0;
+          p.A = w.Dp; p.lda = s.M; p.a_bf16 = s.bf16; p.a_kc = 0; p.a_ones_row = -1;
+          p.B = w.Gx + 4 * (e0 - gb) + 3; p.ldb = 4; p.b_bf16 = 0; p.b_nc = 1;
+          if ((rc = splitk2(p, one ? w.dw2m : res_p + ch * s.M)) != EGNN_OK) return rc;
+        }
       }
       if (w.chunk_gh) {
-        if ((rc = gh_products(e0, e1, gb, one ? w.dwd : res_d + ch * s.H, one ? w.dWe : res_e + ch * Lwe)) != EGNN_OK)
+        if ((rc = gh_products(e0, e1, gb, sp ? nullptr : one ? w.dwd : res_d + ch * s.H, one ? w.dWe : res_e + ch * Lwe)) != EGNN_OK)
           return rc;
         if ((rc = node_reduce(e0, e1, ch > 0)) != EGNN_OK) return rc;
       }
     }
-    if (!one) {
+    if (sp) {   // the kernels' partial rows, summed in row order: dW_hl | dW1_mov (adjacent), dw2_mov | dw_d
+      ProfScope ps(EGNN_K_EDGE_WGRAD, st);
+      if ((rc = hip_status(launch_sum_rows(w.atb, s.E > 0 ? w.atb_rows : 0, w.atb_ld, w.dWhl, st))) != EGNN_OK) return rc;
+      if (s.eq && (rc = hip_status(launch_sum_rows(w.dwpart, s.E > 0 ? w.nblk : 0, w.LW, w.dw2m, st))) != EGNN_OK)
+        return rc;
+      if (!one && s.FE > 0 && (rc = hip_status(launch_sum_rows(res_e, nc, Lwe, w.dWe, st))) != EGNN_OK) return rc;
+    } else if (!one) {
       ProfScope ps(EGNN_K_EDGE_WGRAD, st);
       if ((rc = hip_status(launch_sum_rows(res_w, nc, Lw, w.dWhl, st))) != EGNN_OK) return rc;
       if (s.eq) {

@@ -51,7 +51,7 @@ struct FragSet {
   // order the edge kernels use them.  Chunk 2k: rows 32k .. 32k + 31 of the first product's matrix
   // [row block][k slice][part]; chunk 2k + 1 (EGNN): k slice k of the second's [row block][part].
   void* s_fwd;   // W_hl^T (and W1_mov^T): pre2, q
-  void* s_bwd;   // W1_mov and W_hl (EGNN), W_hl by k slices alone (MPNN): g_m, g_a1
+  void* s_bwd;   // right after it: W1_mov and W_hl (EGNN), W_hl by k slices alone (MPNN): g_m, g_a1
   void* s_u;     // W_u [row block][slot slice][part]
 };
 
@@ -104,6 +104,8 @@ struct BwdWs {
   int64_t chunkE;
   int nchunk;
   bool chunk_gh;   // fp32: Gh, Gx, R2 hold one chunk too, reduced per chunk (node sums accumulated in chunk order)
+  // fp32 split kernels: partial rows of the edge factor products ([atb_rows][atb_ld])
+  float* atb; int64_t atb_rows, atb_ld;
   float* chunkres; // [nchunk][chunk_len]: (H + 1) O + (O + 1) M + M (+ H + H F_E with chunk_gh)
   int64_t chunk_len;
 };
@@ -302,6 +304,20 @@ int launch_wide_bwd(const LayerShape& s, const BwdArgs& a, int nblk, hipStream_t
 // fp32 edge kernels on split operands (egnn_f32.hip): H = O = M = 128
 bool f32_split_supported(const LayerShape& s);
 int launch_f32_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
+// The backward stores the factors Dm1, Dga2 (, Dm, Dgq) of edges [32 tile0, 32 ntiles), and per-block partials of
+// dw2_mov | dw_d ([f32_bwd_blocks][M + H], EGNN) to BwdArgs::dwpart, added to them when fbase > 0 (a later chunk,
+// never of more edges than the first).
+int f32_bwd_blocks(int64_t E);
+int launch_f32_bwd(const LayerShape& s, const BwdArgs& a, hipStream_t st);
+// Per range of len edges: [A0 | 1]^T B0 and (two products) [A1 | 1]^T B1, 129 x 128 each, to its row of part
+struct AtbF32Args {
+  const float *A0, *B0, *A1, *B1;   // [K][128]
+  int64_t K, len;
+  float* part; int64_t ldp;         // [ceil(K / len)][ldp]
+  int add;                          // add to part
+};
+int64_t atb_f32_len(int64_t K);
+int launch_atb_f32(AtbF32Args a, int products, hipStream_t st);
 int bwd_tile_edges(const LayerShape& s);
 
 // dPQ[n] = [sum_row Gh | sum_csc Gh] (summed in fp32, stored in the activation dtype);

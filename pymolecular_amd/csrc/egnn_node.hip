@@ -60,11 +60,11 @@ static int prep_blocks(const LayerShape& s) {
 
 static size_t frag_layout(const LayerShape& s, char* base, FragSet* f, size_t off, bool with_bwd) {
   auto take = [&](size_t bytes) { void* p = base ? base + off : nullptr; off = align_up(off + bytes); return p; };
-  const bool sp = f32_split_supported(s) && !with_bwd;
-  if (sp) {   // bf16 parts of the weights
-    const size_t one = 3 * frag_bytes(s.O, s.H, 2);
-    f->s_fwd = take(s.eq ? 2 * one : one);
-    f->s_bwd = nullptr;
+  const bool sp = f32_split_supported(s);
+  if (sp) {   // bf16 parts of the weights, one run of chunks
+    const size_t one = (s.eq ? 2 : 1) * 3 * frag_bytes(s.O, s.H, 2);
+    f->s_fwd = take(with_bwd ? 2 * one : one);
+    f->s_bwd = (with_bwd && f->s_fwd) ? (char*)f->s_fwd + one : nullptr;
     f->s_u = s.NUC ? take(3 * frag_bytes(s.H, s.KU, 2)) : nullptr;
   } else {
     f->s_fwd = f->s_bwd = f->s_u = nullptr;
@@ -73,9 +73,9 @@ static size_t frag_layout(const LayerShape& s, char* base, FragSet* f, size_t of
   f->hlT = own ? take(frag_bytes(s.O, s.H, s.esz)) : nullptr;
   f->movT = own && s.eq ? take(frag_bytes(s.M, s.O, s.esz)) : nullptr;
   f->u = own && s.NUC ? take(frag_bytes(s.H, s.KU, s.esz)) : nullptr;
-  f->mov = (with_bwd && s.eq) ? take(frag_bytes(s.O, s.M, s.esz)) : nullptr;
-  f->hl = with_bwd ? take(frag_bytes(s.H, s.O, s.esz)) : nullptr;
-  f->uT = (with_bwd && s.eq) ? take(frag_bytes(16, s.H, s.esz)) : nullptr;
+  f->mov = (own && with_bwd && s.eq) ? take(frag_bytes(s.O, s.M, s.esz)) : nullptr;
+  f->hl = own && with_bwd ? take(frag_bytes(s.H, s.O, s.esz)) : nullptr;
+  f->uT = (own && with_bwd && s.eq) ? take(frag_bytes(16, s.H, s.esz)) : nullptr;
   f->b2f = (float*)take(sizeof(float) * s.O);
   f->bx1f = (float*)take(sizeof(float) * (s.M + 4));
   f->w2mf = (float*)take(sizeof(float) * (s.M + 4));
@@ -143,7 +143,7 @@ size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w) {
   char* b = (char*)base;
   size_t off = frag_layout(s, b, &w->fr, 0, true);
   auto take = [&](size_t bytes) { void* p = b ? b + off : nullptr; off = align_up(off + bytes); return p; };
-  const bool coop = coop_supported(s), wide = wide_supported(s);
+  const bool coop = coop_supported(s), wide = wide_supported(s), sp = f32_split_supported(s);
   // edge-major factors; the one-wave-per-tile kernel stores one edge chunk of them at a time
   const int64_t E1 = std::max<int64_t>(s.E, 1);
   w->chunkE = (coop || wide) ? E1 : factor_chunk_edges(s);
@@ -155,18 +155,18 @@ size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w) {
   w->Dm = coop ? nullptr : take(EF * s.O * s.esz);
   w->Dgq = (s.eq && !coop) ? take(EF * s.M * s.esz) : nullptr;
   w->Dga2 = coop ? nullptr : take(EF * s.O * s.esz);
-  w->Dp = (s.eq && !coop && !wide) ? take(EF * s.M * s.esz) : nullptr;
+  w->Dp = (s.eq && !coop && !wide && !sp) ? take(EF * s.M * s.esz) : nullptr;
   // the cooperative kernels store Gh / Gx rows for every edge slot of their last tile (32, 64 or 128 edges)
   const size_t Er = coop ? (size_t)cdiv(std::max<int64_t>(s.E, 1), 4 * kTileEdges) * 4 * kTileEdges
                          : w->chunk_gh ? EF : E;
   w->Gh = take(Er * s.H * s.esz);
   w->Gx = (float*)take(Er * 4 * sizeof(float));
-  w->R2 = (coop || wide) ? nullptr : (float*)take(Er * sizeof(float));
+  w->R2 = (coop || wide || sp) ? nullptr : (float*)take(Er * sizeof(float));
   w->geo = ((coop || wide_supported(s)) && s.eq) ? (float*)take(E * 8 * sizeof(float)) : nullptr;
   w->carry = coop_dst_sums(s) ? (float*)take((size_t)cdiv(E1, kTileEdges) * 2 * s.O * sizeof(float)) : nullptr;
   // per-block partials of the cooperative kernels' weight gradients / the wide kernel's dw2_mov | dw_d
-  w->nblk = coop ? coop_bwd_blocks(s) : (wide && s.eq) ? wide_bwd_blocks(s) : 0;
-  w->LW = coop ? coop_dw_len(s) : (wide && s.eq) ? (int64_t)s.M + s.H : 0;
+  w->nblk = coop ? coop_bwd_blocks(s) : !s.eq ? 0 : wide ? wide_bwd_blocks(s) : sp ? f32_bwd_blocks(w->chunkE) : 0;
+  w->LW = coop ? coop_dw_len(s) : ((wide || sp) && s.eq) ? (int64_t)s.M + s.H : 0;
   w->dwpart = w->nblk > 0 ? (float*)take((size_t)w->nblk * w->LW * sizeof(float)) : nullptr;
   w->dPQ = take((size_t)s.N * 2 * s.H * s.esz);
   // split-K partials: largest (splits x M x N) over the weight-gradient GEMMs
@@ -174,22 +174,28 @@ size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w) {
   if (!coop) {   // the factor products run over one chunk of edges at a time, dw_d and dW_e over all
     // (the split length is rounded per K: the shorter last chunk may need more partial rows)
     const int64_t lastE = std::max<int64_t>(s.E, 1) - (int64_t)(w->nchunk - 1) * w->chunkE;
-    for (const int64_t K : {w->chunkE, lastE})
+    for (const int64_t K : {w->chunkE, lastE}) {
+      if (sp) break;   // atb_f32_kernel, its own partial rows
       w->part_elems = std::max<int64_t>({w->part_elems, splitk_parts(s.H + 1, s.O, K, s.bf16), splitk_parts(s.O + 1, s.M, K, s.bf16),
                                          splitk_parts(s.M, 1, K, s.bf16)});
+    }
     // dw_d and dW_e over Gh: all edges at once, or (chunk_gh) one chunk at a time
     const int64_t Ks[2] = {w->chunk_gh ? w->chunkE : s.E, w->chunk_gh ? lastE : s.E};
     for (const int64_t K : Ks)
       w->part_elems = std::max<int64_t>({w->part_elems, splitk_parts(s.H, 1, K, s.bf16),
                                          splitk_parts(s.H, std::max(s.FE, 1), K, s.bf16)});
   }
+  // sp: partial rows [dW_hl ; db2 | dW1_mov ; dbx1] of the edge ranges, kept over the chunks (the first is the longest)
+  w->atb_ld = sp ? (int64_t)(s.H + 1) * s.O + (s.eq ? (int64_t)(s.O + 1) * s.M : 0) : 0;
+  w->atb_rows = sp ? cdiv(w->chunkE, atb_f32_len(w->chunkE)) : 0;
+  w->atb = sp ? (float*)take((size_t)(w->atb_rows * w->atb_ld) * sizeof(float)) : nullptr;
   w->chunk_len = (int64_t)(s.H + 1) * s.O + (int64_t)(s.O + 1) * s.M + s.M +
                  (w->chunk_gh ? (int64_t)s.H + (int64_t)s.H * std::max(s.FE, 1) : 0);
   w->chunkres = (coop || wide || w->nchunk == 1) ? nullptr
                                                  : (float*)take((size_t)w->nchunk * w->chunk_len * sizeof(float));
   w->part = (float*)take((size_t)w->part_elems * sizeof(float));
-  w->dWhl = (float*)take((size_t)(s.H + 1) * s.O * sizeof(float));
-  w->dW1m = (float*)take((size_t)(s.O + 1) * s.M * sizeof(float));
+  w->dWhl = (float*)take((size_t)((s.H + 1) * s.O + (s.O + 1) * s.M) * sizeof(float));   // adjacent: one sum writes both
+  w->dW1m = w->dWhl ? w->dWhl + (size_t)(s.H + 1) * s.O : nullptr;
   w->dw2m = (float*)take((size_t)(s.M + s.H) * sizeof(float));   // dw2_mov | dw_d, one fixed-order sum in the wide path
   w->dwd = w->dw2m + s.M;
   w->dWe = (float*)take((size_t)s.H * std::max(s.FE, 1) * sizeof(float));
@@ -357,11 +363,15 @@ static int prep_impl(const LayerShape& s, const void* w1, const void* w2, const 
     add3(fr.s_fwd, s.O, s.H, kW, 1, w2, s.lin ? s.H : s.O, 1, both, 0);
     if (s.eq) add3(fr.s_fwd, s.M, s.O, kW, 1, w1m, s.lin ? s.O : s.M, 2, both, rows);
     if (s.NUC) add3(fr.s_u, s.H, s.KU, FK_U, 0, w1, s.H, 1, 6 * s.NUC, 0);
+    if (with_bwd) {
+      if (s.eq) add3(fr.s_bwd, s.O, s.M, kWT, 1, w1m, s.lin ? s.O : s.M, 1, both, 0);
+      add3(fr.s_bwd, s.H, s.O, kWT, 1, w2, s.lin ? s.H : s.O, 2, s.eq ? both : 3 * (s.H / 16), s.eq ? rows : 0);
+    }
   }
   add(fr.hlT, s.O, s.H, kW, 1, w2, s.lin ? s.H : s.O);                // A[o][h] = W_hl[h][o]
   if (s.eq) add(fr.movT, s.M, s.O, kW, 1, w1m, s.lin ? s.O : s.M);    // A[m][o] = W1mov[o][m]
   if (s.NUC) add(fr.u, s.H, s.KU, FK_U, 0, w1, s.H);
-  if (with_bwd) {
+  if (with_bwd && !fr.s_fwd) {
     if (s.eq) add(fr.mov, s.O, s.M, kWT, 1, w1m, s.lin ? s.O : s.M);  // A[o][m] = W1mov[o][m]
     add(fr.hl, s.H, s.O, kWT, 1, w2, s.lin ? s.H : s.O);              // A[h][o] = W_hl[h][o]
     if (s.eq) add(fr.uT, 16, s.H, FK_UT, 1, w1, s.H);
