@@ -185,6 +185,10 @@ int launch_gemm2(const Gemm2Args& g, bool compute_bf16, hipStream_t st);
 constexpr int64_t kStreamMinRows = 65536;
 bool stream_gemm_ok(const Gemm2Args& g, bool compute_bf16);
 int launch_stream_gemm(const Gemm2Args& g, hipStream_t st);
+// fp32 products on split bf16 operands (egnn_gemm32.hip), gz splits; launch_gemm2 takes them for fp32 operands
+// with 16-byte rows and N % 4 == 0
+bool gemm_f32s_ok(const Gemm2Args& g);
+int launch_gemm_f32s(const Gemm2Args& g, unsigned gz, hipStream_t st);
 // The node update's MLP in one streaming pass (egnn_stream.hip): bf16, K1 = Hn = Fo = 128, K2 in {0, 128},
 // N >= kNodeFuseFwdMinRows rows (forward) or kStreamMinRows rows (backward).  Forward: pre = [x1 | x2] W1^T + b1, act = SiLU(pre),
 // out = act W2^T + b2 (+ x1).  Backward: dz = (gout W2) * SiLU'(pre), gx = dz W1 (+ gout on the

@@ -84,3 +84,46 @@ def test_extreme_magnitudes():
     case.p["w1_msg"] = (case.p["w1_msg"] * 2.0 ** -9).astype(np.float32)
     check_case(case, "fp32", backward=False)
     torch.cuda.synchronize()
+
+
+def _gemm_case(N, K1, K2, Hn, Fo, res, seed):
+    """egnn_node_fwd / bwd in fp32 against float64: pre = [x1 | x2] W1^T + b1, out = SiLU(pre) W2^T + b2 (+ x1)."""
+    from pymolecular_amd.node_update import node_update
+    g = torch.Generator().manual_seed(seed)
+    mk = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    x1, x2 = mk(N, K1), mk(N, K2) if K2 else None
+    p = [mk(Hn, K1 + K2) / (K1 + K2) ** 0.5, mk(Hn) * 0.1, mk(Fo, Hn) / Hn ** 0.5, mk(Fo) * 0.1]
+    go = mk(N, Fo)
+
+    def run(conv, f):
+        a = conv(x1).requires_grad_()
+        b = None if x2 is None else conv(x2).requires_grad_()
+        lin = [torch.nn.Linear(K1 + K2, Hn), torch.nn.Linear(Hn, Fo)]
+        for m, w, v in zip(lin, p[::2], p[1::2]):
+            m.weight, m.bias = torch.nn.Parameter(conv(w)), torch.nn.Parameter(conv(v))
+        out = f(a, b, *lin)
+        wrt = [t for t in (a, b) if t is not None] + [t for m in lin for t in m.parameters()]
+        return [out.detach()] + list(torch.autograd.grad(out, wrt, conv(go)))
+
+    def ref(a, b, lin1, lin2):
+        y = lin2(torch.nn.functional.silu(lin1(a if b is None else torch.cat([a, b], 1))))
+        return y + a if res else y
+    got = run(lambda t: t.detach().cuda(), lambda a, b, lin1, lin2: node_update(a, b, lin1, lin2, residual=res))
+    want = run(lambda t: t.detach().double(), ref)
+    for k, (u, v) in enumerate(zip(got, want)):
+        err = ((u.double().cpu() - v).norm() / v.norm().clamp(min=1e-30)).item()
+        # sums of up to N products: 2-norm error of a few 2^-24 times sqrt(log-ish growth); 2e-6 is 30 roundings
+        assert err <= 2e-6, (k, err)
+
+
+@pytest.mark.parametrize("N,K1,K2,Hn,Fo,res", [
+    (1, 128, 128, 128, 128, True),       # one row
+    (31, 128, 0, 128, 128, True),        # below a 32-row tile
+    (33, 8, 8, 24, 8, True),             # K of 16 and 24: a slice's tail, columns past N
+    (65, 128, 128, 128, 128, False),
+    (257, 40, 24, 72, 48, False),        # no multiple of a tile anywhere
+    (8200, 128, 128, 128, 128, True),    # 64-row tiles
+    (4099, 136, 120, 256, 136, True),    # concatenation inside a 32-deep slice
+])
+def test_f32_node_products(N, K1, K2, Hn, Fo, res):
+    _gemm_case(N, K1, K2, Hn, Fo, res, N)
