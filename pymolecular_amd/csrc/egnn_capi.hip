@@ -199,7 +199,8 @@ int32_t egnn_fwd(const EgnnDims* dims, const EgnnStrides* strides, const void* h
     ProfScope ps(EGNN_K_FWD_EDGE, st);
     const int r = coop_supported(s) ? launch_coop_fwd(s, a, st)
                   : wide_supported(s) ? launch_wide_fwd(s, a, st)
-                  : f32_split_supported(s) ? launch_f32_fwd(s, a, st) : launch_fwd(s, a, 0, st);
+                  : f32_split_supported(s) ? launch_f32_fwd(s, a, st)
+                  : f32_small_supported(s) ? launch_f32_small_fwd(s, a, st) : launch_fwd(s, a, 0, st);
     if ((rc = hip_status(r)) != EGNN_OK) return rc;
   }
   ProfScope ps(EGNN_K_FWD_FIXUP, st);
@@ -339,7 +340,18 @@ int32_t egnn_bwd(const EgnnDims* dims, const EgnnStrides* strides, const void* h
     }
     return r;
   };
-  if (!coop && !wide) {
+  const bool small = f32_small_supported(s);
+  if (small) {   // every edge weight gradient in the kernel's partial rows; one chunk of Gh, Gx at a time
+    for (int ch = 0; ch < w.nchunk; ++ch) {
+      const int64_t e0 = (int64_t)ch * w.chunkE, e1 = std::min<int64_t>(s.E, e0 + w.chunkE);
+      a.tile0 = e0 / kTileEdges; a.ntiles = cdiv(e1, kTileEdges); a.fbase = a.gbase = e0;
+      {
+        ProfScope ps(EGNN_K_BWD_EDGE, st);
+        if ((rc = hip_status(launch_f32_small_bwd(s, a, st))) != EGNN_OK) return rc;
+      }
+      if ((rc = node_reduce(e0, e1, ch > 0)) != EGNN_OK) return rc;
+    }
+  } else if (!coop && !wide) {
     // one-wave-per-tile kernel, one edge chunk at a time: each chunk's factor products right after
     // its kernel (sums into per-chunk rows, added in chunk order below when there are several); with
     // chunk_gh (fp32) also the products over the chunk's Gh and its node sums, added to the earlier
@@ -438,7 +450,7 @@ int32_t egnn_bwd(const EgnnDims* dims, const EgnnStrides* strides, const void* h
     if (nsplit * g.M * g.N > w.part_elems) return EGNN_ERR_WORKSPACE;
     ProfScope ps(EGNN_K_WGRAD, st);
     if ((rc = hip_status(launch_gemm2_pair(d, g, s.bf16, st))) != EGNN_OK) return rc;
-    if (coop) {   // both sums, stored in the caller's layout by one launch
+    if (coop || small) {   // both sums, stored in the caller's layout by one launch
       GradSumArgs q{};
       q.part0 = w.dwpart; q.nrows0 = s.E > 0 ? w.nblk : 0; q.L0 = w.LW; q.kind0 = kGradCoop;
       q.part1 = w.part; q.nrows1 = nsplit; q.L1 = g.M * g.N; q.kind1 = kGradWn;

@@ -115,6 +115,8 @@ struct BwdWs {
 //    device with the one-wave-per-tile kernel), and a graph of 2 kChunkMinEdges edges or more has at
 //    least two chunks, so the backward's scratch stays a fraction of its per-edge state (the eager
 //    computation holds all of it); the node reduction runs per chunk and accumulates, in chunk order.
+//    The small kernels (f32_small_supported) keep no factors, 272 bytes per edge instead of 1.3 KB: one chunk
+//    up to the budget.
 //  * bf16: the whole graph when its factor rows take at most kFactorBudget bytes, else half of it.
 // Chunks are whole 32-edge tiles.
 constexpr size_t kFactorBudget = size_t(320) << 20;
@@ -313,6 +315,13 @@ int launch_f32_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
 // never of more edges than the first).
 int f32_bwd_blocks(int64_t E);
 int launch_f32_bwd(const LayerShape& s, const BwdArgs& a, hipStream_t st);
+// fp32 kernels on split operands at the reference's widths (egnn_f32s.hip): H = 64, O = M = 32, at most 32 edge-input
+// slots.  The backward makes every edge weight gradient itself: per-block partial rows [f32_small_blocks][LW] in the
+// layout of coop_dw_len to BwdArgs::dwpart, added to them when fbase > 0 (as launch_f32_bwd); it stores Gh and Gx.
+bool f32_small_supported(const LayerShape& s);
+int f32_small_blocks(int64_t E);
+int launch_f32_small_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
+int launch_f32_small_bwd(const LayerShape& s, const BwdArgs& a, hipStream_t st);
 // Per range of len edges: [A0 | 1]^T B0 and (two products) [A1 | 1]^T B1, 129 x 128 each, to its row of part
 struct AtbF32Args {
   const float *A0, *B0, *A1, *B1;   // [K][128]

@@ -129,10 +129,11 @@ int64_t factor_chunk_edges(const LayerShape& s) {
   const size_t factors = (size_t)(s.H + 2 * s.O + (s.eq ? 2 * s.M : 0)) * s.esz;   // Dm1, Dm, Dga2 (, Dgq, Dp)
   const int64_t whole = cdiv(E, kTileEdges) * kTileEdges;
   if (!s.bf16) {   // fp32: factors, Gh, Gx, r^2 per chunk
-    const size_t per_edge = factors + (size_t)s.H * 4 + 4 * sizeof(float) + sizeof(float);
+    const bool small = f32_small_supported(s);
+    const size_t per_edge = (small ? 0 : factors + sizeof(float)) + (size_t)s.H * 4 + 4 * sizeof(float);
     int64_t n = (int64_t)cdiv((int64_t)((size_t)E * per_edge), (int64_t)kChunkBudget);
     n = std::min<int64_t>(n, std::max<int64_t>(1, E / kChunkFillEdges));   // chunks that fill the device
-    if (E >= 2 * kChunkMinEdges) n = std::max<int64_t>(n, 2);
+    if (E >= 2 * kChunkMinEdges && !small) n = std::max<int64_t>(n, 2);
     return cdiv(cdiv(E, std::max<int64_t>(n, 1)), kTileEdges) * kTileEdges;
   }
   if ((size_t)E * factors <= kFactorBudget) return whole;
@@ -144,6 +145,7 @@ size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w) {
   size_t off = frag_layout(s, b, &w->fr, 0, true);
   auto take = [&](size_t bytes) { void* p = b ? b + off : nullptr; off = align_up(off + bytes); return p; };
   const bool coop = coop_supported(s), wide = wide_supported(s), sp = f32_split_supported(s);
+  const bool small = f32_small_supported(s), own = coop || small;   // own: every edge weight gradient made by the edge kernel
   // edge-major factors; the one-wave-per-tile kernel stores one edge chunk of them at a time
   const int64_t E1 = std::max<int64_t>(s.E, 1);
   w->chunkE = (coop || wide) ? E1 : factor_chunk_edges(s);
@@ -151,27 +153,27 @@ size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w) {
   w->chunk_gh = !coop && !wide && !s.bf16;   // fp32: Gh, Gx, R2 per chunk as well
   const size_t E = (size_t)E1, EF = (size_t)w->chunkE;
   w->PQ = take((size_t)s.N * 2 * s.H * s.esz);
-  w->Dm1 = coop ? nullptr : take(EF * s.H * s.esz);
-  w->Dm = coop ? nullptr : take(EF * s.O * s.esz);
-  w->Dgq = (s.eq && !coop) ? take(EF * s.M * s.esz) : nullptr;
-  w->Dga2 = coop ? nullptr : take(EF * s.O * s.esz);
-  w->Dp = (s.eq && !coop && !wide && !sp) ? take(EF * s.M * s.esz) : nullptr;
+  w->Dm1 = own ? nullptr : take(EF * s.H * s.esz);
+  w->Dm = own ? nullptr : take(EF * s.O * s.esz);
+  w->Dgq = (s.eq && !own) ? take(EF * s.M * s.esz) : nullptr;
+  w->Dga2 = own ? nullptr : take(EF * s.O * s.esz);
+  w->Dp = (s.eq && !own && !wide && !sp) ? take(EF * s.M * s.esz) : nullptr;
   // the cooperative kernels store Gh / Gx rows for every edge slot of their last tile (32, 64 or 128 edges)
   const size_t Er = coop ? (size_t)cdiv(std::max<int64_t>(s.E, 1), 4 * kTileEdges) * 4 * kTileEdges
                          : w->chunk_gh ? EF : E;
   w->Gh = take(Er * s.H * s.esz);
   w->Gx = (float*)take(Er * 4 * sizeof(float));
-  w->R2 = (coop || wide || sp) ? nullptr : (float*)take(Er * sizeof(float));
+  w->R2 = (own || wide || sp) ? nullptr : (float*)take(Er * sizeof(float));
   w->geo = ((coop || wide_supported(s)) && s.eq) ? (float*)take(E * 8 * sizeof(float)) : nullptr;
   w->carry = coop_dst_sums(s) ? (float*)take((size_t)cdiv(E1, kTileEdges) * 2 * s.O * sizeof(float)) : nullptr;
   // per-block partials of the cooperative kernels' weight gradients / the wide kernel's dw2_mov | dw_d
-  w->nblk = coop ? coop_bwd_blocks(s) : !s.eq ? 0 : wide ? wide_bwd_blocks(s) : sp ? f32_bwd_blocks(w->chunkE) : 0;
-  w->LW = coop ? coop_dw_len(s) : ((wide || sp) && s.eq) ? (int64_t)s.M + s.H : 0;
+  w->nblk = coop ? coop_bwd_blocks(s) : small ? f32_small_blocks(w->chunkE) : !s.eq ? 0 : wide ? wide_bwd_blocks(s) : sp ? f32_bwd_blocks(w->chunkE) : 0;
+  w->LW = own ? coop_dw_len(s) : ((wide || sp) && s.eq) ? (int64_t)s.M + s.H : 0;
   w->dwpart = w->nblk > 0 ? (float*)take((size_t)w->nblk * w->LW * sizeof(float)) : nullptr;
   w->dPQ = take((size_t)s.N * 2 * s.H * s.esz);
   // split-K partials: largest (splits x M x N) over the weight-gradient GEMMs
   w->part_elems = splitk_parts(s.F + 1, 2 * s.H, s.N, s.bf16);
-  if (!coop) {   // the factor products run over one chunk of edges at a time, dw_d and dW_e over all
+  if (!own) {   // the factor products run over one chunk of edges at a time, dw_d and dW_e over all
     // (the split length is rounded per K: the shorter last chunk may need more partial rows)
     const int64_t lastE = std::max<int64_t>(s.E, 1) - (int64_t)(w->nchunk - 1) * w->chunkE;
     for (const int64_t K : {w->chunkE, lastE}) {
@@ -191,7 +193,7 @@ size_t bwd_ws_layout(const LayerShape& s, void* base, BwdWs* w) {
   w->atb = sp ? (float*)take((size_t)(w->atb_rows * w->atb_ld) * sizeof(float)) : nullptr;
   w->chunk_len = (int64_t)(s.H + 1) * s.O + (int64_t)(s.O + 1) * s.M + s.M +
                  (w->chunk_gh ? (int64_t)s.H + (int64_t)s.H * std::max(s.FE, 1) : 0);
-  w->chunkres = (coop || wide || w->nchunk == 1) ? nullptr
+  w->chunkres = (own || wide || w->nchunk == 1) ? nullptr
                                                  : (float*)take((size_t)w->nchunk * w->chunk_len * sizeof(float));
   w->part = (float*)take((size_t)w->part_elems * sizeof(float));
   w->dWhl = (float*)take((size_t)((s.H + 1) * s.O + (s.O + 1) * s.M) * sizeof(float));   // adjacent: one sum writes both

@@ -127,3 +127,37 @@ def _gemm_case(N, K1, K2, Hn, Fo, res, seed):
 ])
 def test_f32_node_products(N, K1, K2, Hn, Fo, res):
     _gemm_case(N, K1, K2, Hn, Fo, res, N)
+
+
+@pytest.mark.parametrize("eq", [True, False])
+@pytest.mark.parametrize("kind", ["one", "15", "16", "17", "32", "33", "ones", "halves", "long"])
+def test_small_width_tile_edges(kind, eq):
+    """H = 64, O = M = 32: whole 32-edge tiles per wave in the forward, 16 edges in the backward."""
+    degs = _degrees(kind) + [0] * 5
+    rowptr, col = random_csr(len(degs), degs, seed=len(degs))
+    check_case(Case(rowptr, col, 32, 16, 64, 32, 32, seed=41, eq=eq, mean_agg=eq), "fp32")
+
+
+@pytest.mark.parametrize("eq,fe", [(True, 0), (True, 8), (True, 24), (True, 32), (False, 0), (False, 8), (False, 24),
+                                   (False, 32), (False, 40)])
+@pytest.mark.parametrize("linear", [False, True])
+def test_small_width_edge_slots(eq, fe, linear):
+    """Edge-input slots up to the 32 the small kernels hold and beyond (the general kernels), both weight layouts."""
+    degs = _degrees("halves")
+    rowptr, col = random_csr(len(degs), degs, seed=3)
+    perm = np.random.Generator(np.random.PCG64(3)).permutation(len(col))
+    case = Case(rowptr, col, 48, fe, 64, 32, 32, seed=42, eq=eq, edge_ids=perm)
+    res, gref = run_fused(case, "fp32", linear=linear), case.backward_ref(False)
+    ref = case.forward_ref(False)
+    errs = {"msg": orc.normwise_rel_err(res["out_msg"], ref[0])}
+    for k, v in gref.items():
+        if v is not None and res["grads"].get(k) is not None:
+            errs[k] = orc.normwise_rel_err(res["grads"][k].reshape(v.shape), v)
+    assert all(e <= 1e-5 for e in errs.values()), errs
+
+
+def test_small_width_many_tiles_per_wave():
+    """More edges than one pass of the grid (512 blocks of 64 edges), so every wave accumulates several times."""
+    degs = np.full(3000, 29)
+    rowptr, col = random_csr(len(degs), degs, seed=6)
+    check_case(Case(rowptr, col, 32, 16, 64, 32, 32, seed=43, bias=False), "fp32")
