@@ -654,6 +654,8 @@ __global__ __launch_bounds__(kAtbThreads, 2) void atb_f32_kernel(AtbF32Args a) {
   const float* B = blockIdx.y ? a.B1 : a.B0;
   const int64_t kb = (int64_t)blockIdx.x * a.len;
   const int64_t ke = kb + a.len < a.K ? kb + a.len : a.K;
+  const uint32_t flip = (blockIdx.x & 1) << 31;   // every other range (flip_sign)
+  const float sgn = flip ? -1.0f : 1.0f;
   const int row = tid >> 5, q4 = 4 * (tid & 31);   // the thread's rows row, row + 16 of a slice, columns q4 .. + 3
 
   struct Regs { f32x4 a[2], b[2]; };
@@ -671,7 +673,7 @@ __global__ __launch_bounds__(kAtbThreads, 2) void atb_f32_kernel(AtbF32Args a) {
   f32x4 ones = zero4();
   auto store = [&](int buf, const Regs& r) {
     bf16* base = s_ab + buf * 6 * kAtbPlane + q4;
-    const Chunk3 ca = split_chunk(r.a[0], r.a[1]), cb = split_chunk(r.b[0], r.b[1]);
+    const Chunk3 ca = split_chunk(r.a[0], r.a[1]), cb = split_chunk(flip_sign(r.b[0], flip), flip_sign(r.b[1], flip));
     auto put = [&](int plane, const bf16x8& v) {
       bf16* p = base + plane * kAtbPlane + row * kAtbPitch;
       *reinterpret_cast<bf16x4*>(p) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
@@ -726,7 +728,7 @@ __global__ __launch_bounds__(kAtbThreads, 2) void atb_f32_kernel(AtbF32Args a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float* o = P + (64 * wm + 16 * i + 4 * g + r) * 128 + 32 * wn + 16 * j + c;
-        const float v = hi[i][j][r] + lo[i][j][r];
+        const float v = sgn * (hi[i][j][r] + lo[i][j][r]);
         *o = a.add ? *o + v : v;
       }
   float* s = (float*)s_ab;   // [16][128] sums of the thread rows

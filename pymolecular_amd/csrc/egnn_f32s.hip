@@ -297,6 +297,12 @@ __device__ __forceinline__ void mma16(f32x4& acc, const bf16x4& a, const bf16x4&
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), acc, 0, 0, 0);
 }
+// v with the sign bits of flip (0 or 0x80008000) changed
+__device__ __forceinline__ bf16x4 flip4(const bf16x4& v, uint32_t flip) {
+  const u32x2 x = __builtin_bit_cast(u32x2, v);
+  return __builtin_bit_cast(bf16x4, u32x2{x[0] ^ flip, x[1] ^ flip});
+}
+__device__ __forceinline__ Quad3 flip3(const Quad3& v, uint32_t flip) { return Quad3{flip4(v.p0, flip), flip4(v.p1, flip), flip4(v.p2, flip)}; }
 __device__ __forceinline__ void mma3e(f32x4& acc0, f32x4& acc1, const Quad3& a, const Quad3& b, const Quad3& d) {
   mma16(acc0, a.p2, b.p0);
   mma16(acc1, a.p2, d.p0);
@@ -373,6 +379,8 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
 
   const int64_t ebeg = a.tile0 * kTileEdges, eend = a.ntiles * kTileEdges < E ? a.ntiles * kTileEdges : E;
   const int64_t step = (int64_t)gridDim.x * kW * 16;
+  // every other wave contracts with -B (flip_sign): at 1.9M edges dW1_mov is 2.6e-7 off float64, without it 1.05e-6
+  const uint32_t flip = w & 1 ? 0x80008000u : 0u;
   for (int64_t base = ebeg + ((int64_t)blockIdx.x * kW + w) * 16; base < eend; base += step) {
     const bool valid = base + c < eend;
     const int64_t ee = valid ? base + c : eend - 1;
@@ -483,7 +491,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       sw2 += edge_sums8(pb[0], pb[1], c);
       sbx += edge_sums8(gv[0], gv[1], c);
       wave_sync();
-      const Quad3 B0 = get_slot(sz, 0, c, g), B1 = get_slot(sz, 1, c, g);
+      const Quad3 B0 = flip3(get_slot(sz, 0, c, g), flip), B1 = flip3(get_slot(sz, 1, c, g), flip);
 #pragma unroll
       for (int b = 0; b < 2; ++b) mma3e(gwm[b][0], gwm[b][1], get_slot(sy, b, c, g), B0, B1);
       wave_sync();
@@ -504,7 +512,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       put_slot(sy, l, ga2);
       if constexpr (U) put_slot(sz, l, split_chunk(u.lo, u.hi));
       wave_sync();
-      const Quad3 B0 = get_slot(sy, 0, c, g), B1 = get_slot(sy, 1, c, g);
+      const Quad3 B0 = flip3(get_slot(sy, 0, c, g), flip), B1 = flip3(get_slot(sy, 1, c, g), flip);
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb) mma3e(gwh[hb][0], gwh[hb][1], get_slot(sx + (hb >> 1) * kSlot, hb & 1, c, g), B0, B1);
       wave_sync();
@@ -529,7 +537,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
     }
     if constexpr (U) {
       wave_sync();
-      const Quad3 B0 = get_slot(sz, 0, c, g), B1 = get_slot(sz, 1, c, g);
+      const Quad3 B0 = flip3(get_slot(sz, 0, c, g), flip), B1 = flip3(get_slot(sz, 1, c, g), flip);
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb) mma3e(gwu[hb][0], gwu[hb][1], get_slot(sx + (hb >> 1) * kSlot, hb & 1, c, g), B0, B1);
       wave_sync();
@@ -553,6 +561,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
   for (int q = 0; q < kW; ++q) {
     if (w == q) {
       auto add = [&](int i, float v) { sum[i] = q ? sum[i] + v : v; };
+      const float sgn = flip ? -1.0f : 1.0f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -560,12 +569,12 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int row = 16 * i + 4 * g + r;
-            add(row * O + 16 * j + c, gwh[i][j][r]);
-            if (EQ && i < 2) add(oM + row * M + 16 * j + c, gwm[i < 2 ? i : 0][j][r]);
+            add(row * O + 16 * j + c, sgn * gwh[i][j][r]);
+            if (EQ && i < 2) add(oM + row * M + 16 * j + c, sgn * gwm[i < 2 ? i : 0][j][r]);
             if constexpr (U) {
               const int slot = 8 * (c >> 2) + 4 * j + (c & 3);
-              if (slot < FE) add(oE + row * FE + slot, gwu[i][j][r]);
-              else if (EQ && slot == FE) add(oE + H * FE + row, gwu[i][j][r]);
+              if (slot < FE) add(oE + row * FE + slot, sgn * gwu[i][j][r]);
+              else if (EQ && slot == FE) add(oE + H * FE + row, sgn * gwu[i][j][r]);
             }
           }
       if (!(c & 1)) {

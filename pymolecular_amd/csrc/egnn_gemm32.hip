@@ -83,6 +83,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
   const float* A2 = (const float*)g.A2;
   const float* B = (const float*)g.B;
 
+  const uint32_t flip = g.partial ? (blockIdx.z & 1) << 31 : 0u;   // every other K range (flip_sign)
+  const float sgn = flip ? -1.0f : 1.0f;
+
   struct Regs { f32x4 a[TA::nv], b[TB::nv]; };
   auto load = [&](int64_t k0, Regs& r) {
     if (k0 >= kend) return;   // uniform
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
       for (int i = 0; i < TA::nv; ++i) TA::put(sa, i, r[u].a[i]);
 #pragma unroll
       for (int i = 0; i < TB::nv; ++i) {
-        TB::put(sb, i, r[u].b[i]);
+        TB::put(sb, i, flip_sign(r[u].b[i], flip));
         if constexpr (FOLD) ones += r[u].b[i];
       }
       load(k + kRing * kBK, r[u]);
@@ -178,7 +181,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
       if (n >= g.N) continue;
       f32x4 v = hi[i][j] + lo[i][j];
       if (g.partial) {
-        *reinterpret_cast<f32x4*>(g.partial + ((int64_t)blockIdx.z * g.M + m) * g.N + n) = v;
+        *reinterpret_cast<f32x4*>(g.partial + ((int64_t)blockIdx.z * g.M + m) * g.N + n) = sgn * v;
         continue;
       }
       if (g.bias) {

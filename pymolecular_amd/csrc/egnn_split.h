@@ -81,6 +81,16 @@ __device__ __forceinline__ void mma3x2(f32x4* hi, f32x4* lo, const Chunk3& a, co
   mma(lo[1], d.p0, b.p1);
 }
 
+// The matrix instruction drops the low bits of its sums towards one side, so the errors of many partial sums of one
+// result add up instead of averaging out.  Reductions over edges or nodes therefore contract with -B in every other
+// part and subtract: flip is the sign bit to change in B, sgn the factor of the part's result.
+__device__ __forceinline__ f32x4 flip_sign(const f32x4& v, uint32_t flip) {
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = bitsf(fbits(v[i]) ^ flip);
+  return r;
+}
+
 // SiLU of the fp32 path: e^-x as 2^t (1 + d ln 2) with t = fl(-x log2 e) and d its rounding error (the
 // product's by fma, and log2 e's own), so the exponential keeps the accuracy of v_exp_f32 (1 ulp) for every x.
 // x is clamped in the exponent only, where the sigmoid is 0 or 1 to fp32 precision: an infinite x then gives
