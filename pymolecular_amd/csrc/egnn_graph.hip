@@ -10,11 +10,14 @@
 //    (squared distance, index): kNN keeps the first min(k, n - 1); the radius
 //    graph keeps the first max_nb and drops those farther than the cutoff, which
 //    is the first min(max_nb, #{j : d^2 <= cutoff^2}) of the same order.
-// One wave per node: each lane holds CPL candidates (j = lane + 64 c) sorted by
-// that order, m rounds of a wave-wide minimum over the lanes' heads pick the
-// row, and a bitonic sort across the lanes puts the picked indices in ascending
-// order.  A count pass, a scan and a fill pass give the CSR.  Integer and
-// comparison work only after the distances: bit-exact, no atomics.
+// One wave per node: each lane holds CPL candidates (j = lane + 64 c) by their distance rounded to fp32 (a
+// monotone key, 32-bit order as unsigned), and a bitwise search with ballots finds the key of the m-th nearest: at
+// most 31 steps of CPL compares, usually about 20 (it ends when a key separates m candidates).  Candidates that tie
+// with that key in fp32 are ordered by (d^2, index) in fp64, so the selection is exact.  The selected lanes then
+// store in (c, lane) order, which is ascending index order.  A count pass (kNN: from the segment sizes alone), a
+// scan and a fill pass give the CSR.  Bit-exact, no atomics.
+// Measured (37 chains of 301, k = 30): fill pass about 70 -> 20 us against m rounds of a wave-wide
+// minimum, count pass about 24 -> 5 us.
 #include <hipcub/hipcub.hpp>
 #include "egnn_device.h"
 #include "egnn_internal.h"
@@ -22,12 +25,14 @@
 namespace egnn {
 namespace {
 
+constexpr int kMaxSeg = 64 * 32;   // largest segment
+
 struct GraphArgs {
   const double* pos;      // [N][3]
   int64_t N;
   const int32_t* seg_ptr; // [n_seg + 1]
   int n_seg;
-  int max_seg;            // largest segment the launch was sized for (64 * CPL at most)
+  int max_seg;            // largest segment the caller allows (kMaxSeg at most)
   int mode;               // 0: kNN, 1: radius
   int k;                  // kNN: neighbours per node; radius: max_nb
   double c2;              // radius: cutoff^2 (rounded as the host rounds it)
@@ -48,97 +53,142 @@ __device__ __forceinline__ bool before(double d1, int j1, double d2, int j2) {
   return d1 < d2 || (d1 == d2 && j1 < j2);
 }
 
-template <int CPL>
-__global__ __launch_bounds__(256) void segment_graph_kernel(GraphArgs a, int fill) {
-  const int l = threadIdx.x & 63;
-  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (i >= a.N) return;   // whole waves: N is covered by waves, a wave's lanes share i
-  // the segment of node i: last s with seg_ptr[s] <= i
-  int lo = 0, hi = a.n_seg;
+// the segment of node i: [b, b + n); false (and the error flag) when there is none or it is too large
+__device__ __forceinline__ bool segment_of(const GraphArgs& a, int64_t i, int& b, int& n) {
+  int lo = 0, hi = a.n_seg;   // last s with seg_ptr[s] <= i
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (a.seg_ptr[mid] <= i) lo = mid; else hi = mid;
   }
-  const int b = a.seg_ptr[lo], n = a.seg_ptr[lo + 1] - b;
-  if (b > i || i >= (int64_t)b + n || n > a.max_seg || n > 64 * CPL || (int64_t)b + n > a.N) {
-    if (l == 0) a.err[0] = 1;
+  b = a.seg_ptr[lo];
+  n = a.seg_ptr[lo + 1] - b;
+  return !(b > i || i >= (int64_t)b + n || n > a.max_seg || n > kMaxSeg || (int64_t)b + n > a.N || b < 0);
+}
+
+// kNN row lengths: one thread per node
+__global__ __launch_bounds__(256) void knn_count_kernel(GraphArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.N) return;
+  int b, n;
+  if (!segment_of(a, i, b, n)) {
+    a.err[0] = 1;
+    a.cnt[i] = 0;
     return;
   }
+  a.cnt[i] = min(a.k, n - 1);
+}
+
+constexpr uint32_t kNoKey = 0xffffffffu;
+template <int CPL, bool FILL>
+__device__ __forceinline__ void graph_row(const GraphArgs& a, int64_t i, int b, int n, int l) {
   const double xi[3] = {a.pos[i * 3], a.pos[i * 3 + 1], a.pos[i * 3 + 2]};
-  double kd[CPL];
-  int kj[CPL];
-  int within = 0;
+  uint32_t key[CPL];
+  int total = 0;
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
     const int q = l + 64 * c;
-    const int64_t j = (int64_t)b + q;
-    if (q < n && j != i) {
-      kd[c] = seg_dist2(xi, a.pos + j * 3);
-      kj[c] = (int)j;
-      within += (a.mode == 1 && kd[c] <= a.c2) ? 1 : 0;
-    } else {
-      kd[c] = __builtin_inf();
-      kj[c] = 0x7fffffff;
+    key[c] = kNoKey;
+    if (q < n && b + q != i) {
+      const double d = seg_dist2(xi, a.pos + ((int64_t)b + q) * 3);
+      if (a.mode == 0 || d <= a.c2) key[c] = __builtin_bit_cast(uint32_t, (float)d) & 0x7fffffffu;
     }
+    total += __popcll(__ballot(key[c] != kNoKey));
   }
-  // row length
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) within += __shfl_xor(within, off, 64);
-  const int m = a.mode == 0 ? min(a.k, n - 1) : min(a.k, within);
-  if (!fill) {
+  const int m = min(a.k, total);   // row length
+  if constexpr (!FILL) {
     if (l == 0) a.cnt[i] = m;
     return;
   }
-  // the lane's candidates in (d, j) order: odd-even transposition sort, static indices
+  uint32_t sel = 0;   // bit c: candidate c of the lane is in the row
+  if (m == total) {
 #pragma unroll
-  for (int p = 0; p < CPL; ++p) {
+    for (int c = 0; c < CPL; ++c) sel |= (key[c] != kNoKey ? 1u : 0u) << c;
+  } else {
+    // the largest T with fewer than m keys below it is the key of the m-th
+    uint32_t T = 0;
+    int below = 0;
+    bool exact = false;
+    for (int bit = 30; bit >= 0 && !exact; --bit) {
+      const uint32_t t = T | (1u << bit);
+      int cnt = 0;
 #pragma unroll
-    for (int c = p & 1; c + 1 < CPL; c += 2) {
-      if (before(kd[c + 1], kj[c + 1], kd[c], kj[c])) {
-        const double td = kd[c]; kd[c] = kd[c + 1]; kd[c + 1] = td;
-        const int tj = kj[c]; kj[c] = kj[c + 1]; kj[c + 1] = tj;
+      for (int c = 0; c < CPL; ++c) cnt += __popcll(__ballot(key[c] < t));
+      if (cnt < m) {
+        T = t;
+        below = cnt;
+      } else if (cnt == m) {
+        T = t;
+        exact = true;
+      }
+    }
+    int ties = 0;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      sel |= (key[c] < T ? 1u : 0u) << c;
+      ties += __popcll(__ballot(key[c] == T));
+    }
+    if (!exact) {
+      int need = m - below;   // of the ties
+      if (need == ties) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) sel |= (key[c] == T ? 1u : 0u) << c;
+      } else {
+        for (; need > 0; --need) {   // the wave-wide first of the remaining ties by (d, j)
+          double bd = __builtin_inf();
+          int bj = 0x7fffffff;
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) {
+            if (key[c] != T || ((sel >> c) & 1u)) continue;
+            const int j = b + l + 64 * c;
+            double d = seg_dist2(xi, a.pos + (int64_t)j * 3);
+            if (d != d) d = __builtin_inf();
+            if (before(d, j, bd, bj)) { bd = d; bj = j; }
+          }
+#pragma unroll
+          for (int off = 32; off > 0; off >>= 1) {
+            const double od = __shfl_xor(bd, off, 64);
+            const int oj = __shfl_xor(bj, off, 64);
+            if (before(od, oj, bd, bj)) { bd = od; bj = oj; }
+          }
+          const int q = bj - b;
+          if ((q & 63) == l) sel |= 1u << (q >> 6);
+        }
       }
     }
   }
-  // m rounds: the wave-wide first of the lanes' heads goes to lane r; its lane drops it
-  int mine = 0x7fffffff;
-  for (int r = 0; r < m; ++r) {
-    double bd = kd[0];
-    int bj = kj[0];
+  int at = a.rowptr[i];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const double od = __shfl_xor(bd, off, 64);
-      const int oj = __shfl_xor(bj, off, 64);
-      if (before(od, oj, bd, bj)) { bd = od; bj = oj; }
-    }
-    if (l == r) mine = bj;
-    if (kj[0] == bj) {   // indices are distinct: exactly one lane
-#pragma unroll
-      for (int c = 0; c + 1 < CPL; ++c) { kd[c] = kd[c + 1]; kj[c] = kj[c + 1]; }
-      kd[CPL - 1] = __builtin_inf();
-      kj[CPL - 1] = 0x7fffffff;
-    }
+  for (int c = 0; c < CPL; ++c) {
+    const bool s = (sel >> c) & 1u;
+    const uint64_t mask = __ballot(s);
+    if (s) a.col[(int64_t)at + __popcll(mask & ((1ull << l) - 1ull))] = b + l + 64 * c;
+    at += __popcll(mask);
   }
-  // ascending indices across the lanes (bitonic; lanes past m hold the largest int)
-#pragma unroll
-  for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      const int other = __shfl_xor(mine, stride, 64);
-      const bool up = (l & size) == 0, lower = (l & stride) == 0;
-      mine = (lower == up) ? min(mine, other) : max(mine, other);
-    }
-  }
-  if (l < m) a.col[(int64_t)a.rowptr[i] + l] = mine;
 }
 
-__global__ void graph_zero_kernel(int32_t* p) { p[0] = 0; }
-
-template <int CPL>
-void launch_segment_graph(const GraphArgs& a, int fill, hipStream_t st) {
-  const unsigned blocks = (unsigned)cdiv(a.N, 4);
-  hipLaunchKernelGGL((segment_graph_kernel<CPL>), dim3(blocks), dim3(256), 0, st, a, fill);
+// one wave per node; each takes the smallest of the compiled candidate counts that holds its segment
+template <bool FILL>
+__global__ __launch_bounds__(256) void segment_graph_kernel(GraphArgs a) {
+  const int l = threadIdx.x & 63;
+  const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (i >= a.N) return;   // whole waves: N is covered by waves, a wave's lanes share i
+  int b, n;
+  if (!segment_of(a, i, b, n)) {
+    if (l == 0) {
+      a.err[0] = 1;
+      if (!FILL) a.cnt[i] = 0;
+    }
+    return;
+  }
+  if (n <= 64) graph_row<1, FILL>(a, i, b, n, l);
+  else if (n <= 128) graph_row<2, FILL>(a, i, b, n, l);
+  else if (n <= 256) graph_row<4, FILL>(a, i, b, n, l);
+  else if (n <= 512) graph_row<8, FILL>(a, i, b, n, l);
+  else if (n <= 1024) graph_row<16, FILL>(a, i, b, n, l);
+  else graph_row<32, FILL>(a, i, b, n, l);
 }
+
+__global__ void graph_zero_kernel(int32_t* p, int32_t* q) { p[0] = q[0] = 0; }
 
 struct GraphTmp {
   int32_t* cnt;
@@ -164,7 +214,7 @@ int32_t segment_graph(const double* pos, int64_t N, const int32_t* seg_ptr, int3
                       int32_t k, double c2, int32_t* rowptr, int32_t* col, int64_t col_capacity, void* tmp,
                       size_t tmp_bytes, int64_t* n_edges, hipStream_t st) {
   if (!pos || !seg_ptr || !rowptr || !col || !tmp || !n_edges) return EGNN_ERR_NULL;
-  if (N < 1 || N > (int64_t)INT32_MAX - 1 || n_seg < 1 || max_seg < 1 || max_seg > 64 * 32 || k < 1 || k > 64)
+  if (N < 1 || N > (int64_t)INT32_MAX - 1 || n_seg < 1 || max_seg < 1 || max_seg > kMaxSeg || k < 1 || k > 64)
     return EGNN_ERR_DIMS;
   if (col_capacity < N * (int64_t)k) return EGNN_ERR_WORKSPACE;
   if ((uintptr_t)pos & 7) return EGNN_ERR_ALIGN;
@@ -174,28 +224,18 @@ int32_t segment_graph(const double* pos, int64_t N, const int32_t* seg_ptr, int3
   GraphArgs a{};
   a.pos = pos; a.N = N; a.seg_ptr = seg_ptr; a.n_seg = n_seg; a.max_seg = max_seg; a.mode = mode; a.k = k; a.c2 = c2;
   a.cnt = t.cnt; a.rowptr = rowptr; a.col = col; a.err = t.err;
-  const int cpl = max_seg <= 64 ? 1 : max_seg <= 128 ? 2 : max_seg <= 256 ? 4 : max_seg <= 512 ? 8 : max_seg <= 1024 ? 16 : 32;
-  auto launch = [&](int fill) {
-    switch (cpl) {
-      case 1: launch_segment_graph<1>(a, fill, st); break;
-      case 2: launch_segment_graph<2>(a, fill, st); break;
-      case 4: launch_segment_graph<4>(a, fill, st); break;
-      case 8: launch_segment_graph<8>(a, fill, st); break;
-      case 16: launch_segment_graph<16>(a, fill, st); break;
-      default: launch_segment_graph<32>(a, fill, st); break;
-    }
-  };
-  hipLaunchKernelGGL(graph_zero_kernel, dim3(1), dim3(1), 0, st, t.err);
-  launch(0);
+  const dim3 wgrid((unsigned)cdiv(a.N, 4));
+  hipLaunchKernelGGL(graph_zero_kernel, dim3(1), dim3(1), 0, st, t.err, rowptr);
+  if (mode == 0) hipLaunchKernelGGL(knn_count_kernel, dim3((unsigned)cdiv(a.N, 256)), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((segment_graph_kernel<false>), wgrid, dim3(256), 0, st, a);
   size_t cb = t.cub_bytes;
   if (hipcub::DeviceScan::InclusiveSum(t.cub, cb, t.cnt, rowptr + 1, (int)N, st) != hipSuccess) return EGNN_ERR_HIP;
-  hipLaunchKernelGGL(graph_zero_kernel, dim3(1), dim3(1), 0, st, rowptr);
   int32_t host[2] = {0, 0};
   if (hipMemcpyAsync(&host[0], t.err, sizeof(int32_t), hipMemcpyDeviceToHost, st) != hipSuccess) return EGNN_ERR_HIP;
   if (hipMemcpyAsync(&host[1], rowptr + N, sizeof(int32_t), hipMemcpyDeviceToHost, st) != hipSuccess) return EGNN_ERR_HIP;
   if (hipStreamSynchronize(st) != hipSuccess) return EGNN_ERR_HIP;
   if (host[0]) return EGNN_ERR_DIMS;
-  launch(1);
+  hipLaunchKernelGGL((segment_graph_kernel<true>), wgrid, dim3(256), 0, st, a);
   if (hipGetLastError() != hipSuccess) return EGNN_ERR_HIP;
   *n_edges = host[1];
   return EGNN_OK;

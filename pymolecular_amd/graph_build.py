@@ -20,6 +20,9 @@ from ._capi import check
 
 __all__ = ["knn_graph", "radius_graph"]
 
+# largest segment the kernels take; they check every segment themselves, so the sizes need not come to the host first
+MAX_SEG = 2048
+
 
 def _prep(pos: torch.Tensor, seg_ptr: torch.Tensor):
     if not pos.is_cuda:
@@ -30,11 +33,10 @@ def _prep(pos: torch.Tensor, seg_ptr: torch.Tensor):
     seg = seg_ptr.to(device=pos.device, dtype=torch.int32).contiguous()
     if seg.dim() != 1 or seg.numel() < 2:
         raise ValueError("seg_ptr must hold n_seg + 1 >= 2 offsets")
-    max_seg = int(torch.diff(seg).max().item())
-    return pos, seg, max_seg
+    return pos, seg
 
 
-def _build(fn, pos, seg, max_seg, m, extra):
+def _build(fn, pos, seg, m, extra):
     N = pos.shape[0]
     L = _capi.lib()
     dev = pos.device
@@ -44,7 +46,7 @@ def _build(fn, pos, seg, max_seg, m, extra):
     tmp = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
     ne = ctypes.c_int64(0)
     st = torch.cuda.current_stream(dev).cuda_stream
-    rc = getattr(L, fn)(pos.data_ptr(), N, seg.data_ptr(), seg.numel() - 1, max_seg, *extra, rowptr.data_ptr(),
+    rc = getattr(L, fn)(pos.data_ptr(), N, seg.data_ptr(), seg.numel() - 1, MAX_SEG, *extra, rowptr.data_ptr(),
                         col.data_ptr(), col.numel(), tmp.data_ptr(), nbytes, ctypes.byref(ne), st)
     check(fn, rc)
     return rowptr, col[:ne.value]
@@ -52,11 +54,11 @@ def _build(fn, pos, seg, max_seg, m, extra):
 
 def knn_graph(pos: torch.Tensor, seg_ptr: torch.Tensor, k: int):
     """CSR ``(rowptr, col)`` of each node's ``min(k, n - 1)`` nearest other nodes of its segment."""
-    pos, seg, max_seg = _prep(pos, seg_ptr)
-    return _build("egnn_knn_graph", pos, seg, max_seg, k, (int(k),))
+    pos, seg = _prep(pos, seg_ptr)
+    return _build("egnn_knn_graph", pos, seg, k, (int(k),))
 
 
 def radius_graph(pos: torch.Tensor, seg_ptr: torch.Tensor, cutoff: float, max_nb: int):
     """CSR ``(rowptr, col)`` of each node's nearest ``max_nb`` other nodes of its segment within ``cutoff``."""
-    pos, seg, max_seg = _prep(pos, seg_ptr)
-    return _build("egnn_radius_graph", pos, seg, max_seg, max_nb, (ctypes.c_double(float(cutoff)), int(max_nb)))
+    pos, seg = _prep(pos, seg_ptr)
+    return _build("egnn_radius_graph", pos, seg, max_nb, (ctypes.c_double(float(cutoff)), int(max_nb)))
