@@ -23,6 +23,7 @@ CSRC = PKG / "csrc"
 HEADER = PKG.parent / "include" / "egnn.h"
 LIB = PKG / "libpymolecular_egnn.so"
 STAMP = LIB.with_name(LIB.name + ".srchash")
+EXT = PKG / "_egnn_torch.so"   # the layer's native autograd node (csrc/egnn_torch.cpp), linked to LIB
 OBJ = PKG / "_objs"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -45,7 +46,30 @@ FILE_FLAGS = {
 
 
 def source_files() -> list:
-    return sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.h")) + [HEADER]
+    return sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.cpp")) + sorted(CSRC.glob("*.h")) + [HEADER]
+
+
+def _ext_commands():
+    """(compile, link) of the autograd node: host code against torch's headers, no device code."""
+    import sysconfig
+
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    obj = OBJ / "egnn_torch.o"
+    inc = [f"-I{root / 'include'}", f"-I{root / 'include/torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}",
+           "-I" + os.environ.get("ROCM_PATH", "/opt/rocm") + "/include"]
+    cc = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-w", *inc, "-c",
+          str(CSRC / "egnn_torch.cpp"), "-o", str(obj)]
+    ld = ["g++", "-shared", "-o", str(EXT), str(obj), f"-L{PKG}", "-l:" + LIB.name, f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+          "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    return cc, ld
+
+
+def _run(cmd, what) -> None:
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n" + r.stderr[-6000:])
 
 
 def source_hash() -> str:
@@ -76,7 +100,10 @@ def build(verbose: bool = True) -> Path:
     srcs = sorted(CSRC.glob("*.hip"))
     jobs = min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
     with cf.ThreadPoolExecutor(jobs) as ex:
+        ext_cc, ext_ld = _ext_commands()
+        ext = ex.submit(_run, ext_cc, "compiling egnn_torch.cpp")   # the longest single file
         objs = list(ex.map(_compile, srcs))
+        ext.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -85,6 +112,7 @@ def build(verbose: bool = True) -> Path:
     if STAMP.exists():
         STAMP.unlink()
     os.replace(tmp, LIB)
+    _run(ext_ld, "linking " + EXT.name)
     STAMP.write_text(digest + "\n")
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources (sources sha256 {digest[:16]})")

@@ -157,6 +157,20 @@ def lib() -> ctypes.CDLL:
     return L
 
 
+_ext = None
+
+
+def ext():
+    """The native autograd node of the layer (csrc/egnn_torch.cpp), loaded once; raises if it has not been built."""
+    global _ext
+    if _ext is None:
+        import torch  # noqa: F401  (its libraries, which the module links to)
+        lib()         # built from these sources
+        from . import _egnn_torch
+        _ext = _egnn_torch
+    return _ext
+
+
 PROFILE_ALL = 0xFF   # include/egnn.h EGNN_PROFILE_ALL
 
 

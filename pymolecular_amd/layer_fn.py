@@ -20,10 +20,25 @@ from __future__ import annotations
 
 import torch
 
+from ._capi import ext
 from .fused import _dims, _fused_backward, _fused_forward, _node_proj_buffer, _prep_inputs, get_schedule
 from .node_update import node_update_backward, node_update_forward
 
-__all__ = ["GCLLayerFn"]
+__all__ = ["GCLLayerFn", "gcl_layer"]
+
+
+def gcl_layer(h, coord, edge_attr, row_ptrs, col, perm, e0w, e0b, e2w, e2b, c0w, c0b, c2w, n0w, n0b, n2w, n2b,
+              mean_agg, residual, equivariant):
+    """The layer of :class:`GCLLayerFn`, by the native autograd node (csrc/egnn_torch.cpp: the same library calls,
+    allocations and backward without Python) when no tensor needs a conversion, else by the Python one."""
+    if h.is_cuda and row_ptrs.is_cuda:
+        sched = get_schedule(row_ptrs, col, h.shape[0])
+        out = ext().gcl_layer(h, coord, edge_attr, row_ptrs, col, perm, e0w, e0b, e2w, e2b, c0w, c0b, c2w, n0w, n0b,
+                              n2w, n2b, sched.buf, mean_agg, residual, equivariant)
+        if out is not None:
+            return out
+    return GCLLayerFn.apply(h, coord, edge_attr, row_ptrs, col, perm, e0w, e0b, e2w, e2b, c0w, c0b, c2w, n0w, n0b,
+                            n2w, n2b, mean_agg, residual, equivariant)
 
 
 class GCLLayerFn(torch.autograd.Function):
