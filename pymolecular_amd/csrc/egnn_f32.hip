@@ -36,8 +36,9 @@ __device__ __forceinline__ Chunk3 lds_chunk3(const bf16* frag, int l) {
 struct RowAddr {
   uint32_t lo, hi;
   __device__ __forceinline__ explicit RowAddr(float* p) : lo((uint32_t)(uintptr_t)p), hi((uint32_t)((uintptr_t)p >> 32)) {}
-  __device__ __forceinline__ float* of(int r) const {
-    return (float*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, r) << 32) |
+  // in the global address space: a generic (flat) store also waits for the LDS
+  __device__ __forceinline__ __attribute__((address_space(1))) float* of(int r) const {
+    return (__attribute__((address_space(1))) float*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, r) << 32) |
                     (uint32_t)__builtin_amdgcn_readlane((int)lo, r));
   }
 };
@@ -164,6 +165,9 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
         m1[kc] = split_chunk(y[kc][0], y[kc][1]);
       }
     }
+    // loaded before the gathers, so complete by now: named here, not at each row's store, which would then wait for
+    // every load under way
+    __asm__ __volatile__("" ::"v"(tabv), "v"(am.lo), "v"(am.hi), "v"(ax.lo), "v"(ax.hi), "v"(dx), "v"(dy), "v"(dz));
     // ---- S2 and S3, 32 message features at a time
     f32x4 q[EQ ? M / 16 : 1];
     if constexpr (EQ) {

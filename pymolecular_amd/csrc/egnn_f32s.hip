@@ -212,11 +212,12 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
           acc += v[k];
           ++n;
           if ((ends >> (k0 + k)) & 1u) {
-            float* const om = (float*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mhi, r) << 32) |
+            typedef __attribute__((address_space(1))) float gfloat;
+            gfloat* const om = (gfloat*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mhi, r) << 32) |
                                        (uint32_t)__builtin_amdgcn_readlane((int)mlo, r));
             if (l < O) om[l] = acc;
             if constexpr (EQ) {
-              float* const ox = (float*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)xhi, r) << 32) |
+              gfloat* const ox = (gfloat*)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)xhi, r) << 32) |
                                          (uint32_t)__builtin_amdgcn_readlane((int)xlo, r));
               if (l >= O && l < O + 3) ox[l - O] = a.mean && __builtin_amdgcn_readlane(tabv, r) >= 0 ? acc / (float)n : acc;
             }

@@ -1,0 +1,34 @@
+"""Edge-parallel forward at H = 256 (bf16) at the edges of its tiles and passes, against the oracle."""
+import numpy as np
+import pytest
+
+from tests.cases import Case, random_csr
+from tests.test_f32_split_gpu import _degrees
+from tests.test_fused_gpu import check_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("eq", [True, False])
+@pytest.mark.parametrize("kind", ["one", "15", "17", "32", "33", "ones", "halves", "long"])
+def test_tile_edges(kind, eq):
+    """Tiles of 1 to 32 ranks, rows over tiles, a pass with fewer tiles than the block's waves."""
+    degs = _degrees(kind) + [0] * 5   # sources besides the row itself
+    rowptr, col = random_csr(len(degs), degs, seed=len(degs))
+    check_case(Case(rowptr, col, 256, 8, 256, 256, 256, seed=51, eq=eq, mean_agg=eq), "bf16")
+
+
+@pytest.mark.parametrize("eq,fe", [(True, 0), (True, 24), (True, 32), (True, 56), (False, 8), (False, 32), (False, 40), (False, 64)])
+def test_edge_slots(eq, fe):
+    """One and two 32-slot slices of edge inputs, permuted edge ids."""
+    degs = _degrees("halves")
+    rowptr, col = random_csr(len(degs), degs, seed=3)
+    perm = np.random.Generator(np.random.PCG64(3)).permutation(len(col))
+    check_case(Case(rowptr, col, 64, fe, 256, 256, 256, seed=52, eq=eq, edge_ids=perm), "bf16")
+
+
+def test_many_passes():
+    """More tiles than one pass of the grid (512 blocks of four tiles)."""
+    degs = np.full(2100, 33)
+    rowptr, col = random_csr(len(degs), degs, seed=6)
+    check_case(Case(rowptr, col, 16, 16, 256, 256, 256, seed=53, bias=False), "bf16", backward=False)
