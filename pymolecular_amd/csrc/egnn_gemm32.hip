@@ -8,7 +8,7 @@
 // The product is computed transposed, so a lane holds four consecutive columns of one row and every epilogue
 // access is a 16-byte one.
 // Measured against the fp32-instruction tiles it replaced, per launch: 27 x 256 -> 128 products 16.7 -> 7.1 us,
-// 2,351 rows 20.9 -> 8.2 us, 19,623 rows 36 -> 26 us; [x | 1]^T dz over 2,351 rows 13.9 -> 11 us, over 19,623 rows
+// 2,351 rows 20.9 -> 8.2 us, 19,623 rows 36 -> 23 us; [x | 1]^T dz over 2,351 rows 13.9 -> 11 us, over 19,623 rows
 // 29 -> 21 us.
 #include "egnn_device.h"
 #include "egnn_internal.h"
@@ -251,9 +251,7 @@ int launch_gemm_f32s(const Gemm2Args& g, unsigned gz, hipStream_t st) {
   const unsigned gy = (unsigned)cdiv(g.N, kBN);
   if (g.partial && !g.a_kc && g.b_nc && g.a_ones_row == g.M - 1 && g.M > 1 && (g.M - 1) % 64 == 0) {
     launch_bm<64, true>(g, dim3((unsigned)((g.M - 1) / 64), gy, gz), st);
-  } else if (cdiv(g.M, 64) * gy * (int64_t)gz >= 512) {   // enough blocks for two per CU
-    launch_bm<64, false>(g, dim3((unsigned)cdiv(g.M, 64), gy, gz), st);
-  } else {
+  } else {   // 32-row tiles at every size: three blocks per CU, at 19,623 rows 23 us against 26 us with 64-row tiles
     launch_bm<32, false>(g, dim3((unsigned)cdiv(g.M, 32), gy, gz), st);
   }
   return (int)hipGetLastError();

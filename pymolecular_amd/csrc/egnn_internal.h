@@ -122,6 +122,10 @@ struct BwdWs {
 constexpr size_t kFactorBudget = size_t(320) << 20;
 constexpr size_t kChunkBudget = size_t(256) << 20;
 constexpr int64_t kChunkMinEdges = 4096;
+// H = 128 on split operands: two chunks from here on only.  Below, one chunk (2.6 KB per edge) takes two passes of
+// the backward's grid where two chunks of half the edges take one each and leave it half empty, and saves three
+// launches: at 46k edges 67 + 27 + 12 us (backward, factor products, node sums) against 88 + 41 + 20 us.
+constexpr int64_t kSplitTwoChunks = 65536;
 constexpr int64_t kChunkFillEdges = 6144 * 32;
 int64_t factor_chunk_edges(const LayerShape& s);
 size_t fwd_ws_layout(const LayerShape& s, void* base, FwdWs* w);

@@ -133,7 +133,8 @@ int64_t factor_chunk_edges(const LayerShape& s) {
     const size_t per_edge = (small ? 0 : factors + sizeof(float)) + (size_t)s.H * 4 + 4 * sizeof(float);
     int64_t n = (int64_t)cdiv((int64_t)((size_t)E * per_edge), (int64_t)kChunkBudget);
     n = std::min<int64_t>(n, std::max<int64_t>(1, E / kChunkFillEdges));   // chunks that fill the device
-    if (E >= 2 * kChunkMinEdges && !small) n = std::max<int64_t>(n, 2);
+    const int64_t two = f32_split_supported(s) ? kSplitTwoChunks : 2 * kChunkMinEdges;
+    if (E >= two && !small) n = std::max<int64_t>(n, 2);
     return cdiv(cdiv(E, std::max<int64_t>(n, 1)), kTileEdges) * kTileEdges;
   }
   if ((size_t)E * factors <= kFactorBudget) return whole;
