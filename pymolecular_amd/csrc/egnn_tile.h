@@ -84,39 +84,9 @@ __device__ __forceinline__ bf16x8 chain_edge_major(const bf16* buf, int blk, int
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// Edge-feature tile stored slot-major for the dW_e products: row `slot` holds the tile's 32
-// edges in kappa_chain order, so the B operand of lane (c, g) (edges kappa_chain(g, s) of one
-// slot) is one 16-byte read.  Edge 16 nb + c sits at position 8 (c >> 2) + 4 nb + (c & 3).
-__device__ __forceinline__ void put_ut(bf16* buf, int nb, int c, int g, const bf16x8& u) {
-  bf16* p = buf + 8 * g * TE + 8 * (c >> 2) + 4 * nb + (c & 3);   // slots 8g .. 8g + 7 of the edge
-#pragma unroll
-  for (int s = 0; s < 8; ++s) p[s * TE] = u[s];
-}
-__device__ __forceinline__ bf16x8 get_ut(const bf16* buf, int slot, int g) {
-  return *reinterpret_cast<const bf16x8*>(buf + slot * TE + 8 * g);
-}
-// The A chunk over the tile's 32 edges (kappa_chain) of a C-block transposed to edge-major
-// (transpose_block) that covers only edge block nb: elements 4 nb .. 4 nb + 3, zeros elsewhere.
-// nb must be wave-uniform (a select of whole registers, no per-element moves).
-__device__ __forceinline__ bf16x8 half_edge_chunk(const f32x4& t, int nb) {
-  const u32x2 v = __builtin_bit_cast(u32x2, pack4(t));
-  const u32x4 q = nb ? u32x4{0u, 0u, v[0], v[1]} : u32x4{v[0], v[1], 0u, 0u};
-  return __builtin_bit_cast(bf16x8, q);
-}
-
 __device__ __forceinline__ int rank_of(uint32_t mask, int k) {
   const uint32_t below = (k >= 31) ? 0xffffffffu : ((2u << k) - 1u);
   return __popc(mask & below) - 1;
-}
-// B operand S[edge][rank]: column n = rank 16*rb + c, rows = edges kappa_chain(g, s)
-__device__ __forceinline__ bf16x8 seg_chunk(uint32_t mask, int nvalid, int rb, int c, int g) {
-  bf16x8 r;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const int k = kappa_chain(g, s);
-    r[s] = (k < nvalid && rank_of(mask, k) == 16 * rb + c) ? (bf16)1.0f : (bf16)0.0f;
-  }
-  return r;
 }
 
 // A operand that adds two 4-row halves of a B chunk: A[r][8g + s] = (r == 4g + (s & 3)), so
@@ -226,8 +196,6 @@ __device__ __forceinline__ bf16x8 input_chunk(const bf16* ef, int64_t se, int ei
   }
   return z;
 }
-
-__device__ __forceinline__ uint32_t lo16(unsigned long long b) { return (uint32_t)(b & 0xffffull); }
 
 // A operands from a row-major bf16 matrix W in LDS (row pitch P), K slice kc,
 // lane (c, g) element s <-> k = 32 kc + kappa_chain(g, s):
