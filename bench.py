@@ -18,7 +18,7 @@ edges per second through the fused layer.
 roofline: the dominant edge kernel of the step (the fused backward), its
 time per layer from HIP events recorded on the stream it runs on during the
 timed steps (the library's instrumentation hook; one launch per layer, or
-one per edge chunk of the one-wave-per-tile backward) -- plus, on the paths
+one per edge chunk of the fp32 backward) -- plus, on the paths
 whose backward kernel stores per-edge factors (H = 256, and fp32), the
 weight-gradient products over those factors that finish its work (class
 edge_wgrad) -- and its algorithmic work per layer from the per-edge model of
@@ -28,7 +28,8 @@ the reference formulation:
     B_bwd = E (8 + F s + c + F_E s + 4F + c) + N (4 + F s + 3c + O s + 4F)
 (g = 1 for EGNN, 0 for MPNN; c = 16 g; s = bytes per activation), bounded by
 whichever of HBM (8 TB/s) and MFMA (bf16 2516.6, fp32 157.3 TFLOP/s) takes
-longer for that work.  ``executed`` gives the same kernel's work as this
+longer for that work (the fp32 kernels run their products as bf16 parts and
+are still priced at the fp32 instruction's rate).  ``executed`` gives the same kernel's work as this
 build executes it (projections hoisted to the nodes, scratch traffic).
 ``traffic`` is the measured HBM bytes per launch from the rocprofv3
 FETCH_SIZE / WRITE_SIZE summary under profiles/ when one exists.
@@ -122,9 +123,9 @@ def kernel_work(cls, path, N, E, F, H, O, M, FE, g, s):
         elif path == "wide":  # factors m1, m, g_q, g_a2 stored for the split-K products (dw2_mov, dw_d in the kernel)
             flops = 2 * (g + FE) * H + 4 * H * O + 4 * g * O * M
             per_edge += (H + O + g * M + O) * s
-        else:         # one wave per tile: factors m1, m, g_q, p, g_a2 and r^2 stored for the split-K products
-            flops = 2 * (g + FE) * H + 4 * H * O + 4 * g * O * M
-            per_edge += (H + O + 2 * g * M + O) * s + 4 * g
+        else:                 # fp32 on split operands: the same factors; dw2_mov, dw_d and dW_e in the kernel
+            flops = 4 * (g + FE) * H + 4 * H * O + 4 * g * O * M
+            per_edge += (H + O + g * M + O) * s
         if dst:
             return flops * E, E * (per_edge + H / 4) + N * H * s
         return flops * E, E * per_edge
@@ -141,9 +142,9 @@ def kernel_work(cls, path, N, E, F, H, O, M, FE, g, s):
         if path == "wide":     # [dW_hl; db2], [dW1_mov; dbx1] over the edge factors; dW_e over Gh
             flops = 2 * E * ((H + 1) * O + g * (O + 1) * M + H * FE)
             nbytes = E * ((H + O) * s + g * (O + M) * s + (H * s + FE * s + 4 if FE else 0))
-        elif path == "one":    # the same, plus the dw2_mov and dw_d matrix-vector products over p, Gh and r^2
-            flops = 2 * E * ((H + 1) * O + g * ((O + 1) * M + M + H) + H * FE)
-            nbytes = E * ((H + O) * s + g * ((O + M) * s + M * s + 4 + H * s + 4) + (H * s + FE * s + 4 if FE else 0))
+        elif path == "split":  # [dW_hl; db2], [dW1_mov; dbx1] over the edge factors
+            flops = 2 * E * ((H + 1) * O + g * (O + 1) * M)
+            nbytes = E * ((H + O) * s + g * (O + M) * s)
         return flops, nbytes
     return 0, 0
 
@@ -312,7 +313,7 @@ def run_workload(k, dtype, a, g=None):
 
     s = 2 if dt == torch.bfloat16 else 4
     g1 = 1 if eq else 0
-    path = "coop" if s == 2 and H == 128 and FE + 2 * g1 <= 32 else "wide" if s == 2 and H == 256 else "one"
+    path = "coop" if s == 2 and H == 128 and FE + 2 * g1 <= 32 else "wide" if s == 2 and H == 256 else "split"
     peak_mfma = PEAK["bf16_mfma_tflops"] if s == 2 else PEAK["fp32_mfma_tflops"]
 
     def executed_per_launch(cls, launches_per_step):
@@ -340,7 +341,7 @@ def run_workload(k, dtype, a, g=None):
                                  hbm_frac=by / (per / 1e3) / (PEAK["hbm_gbs"] * 1e9), flops=fl, bytes=by)
     edge_cls = [c for c in ("bwd_edge", "fwd_edge") if c in kern]
     dom = max(edge_cls, key=lambda c: kern[c]["ms_per_launch"] * kern[c]["launches_per_step"])
-    # one layer's launches of the class (one, or one per edge chunk of the one-wave-per-tile backward)
+    # one layer's launches of the class (one, or one per edge chunk of the fp32 backward)
     per_layer = kern[dom]["launches_per_step"] / L
     dur_s = kern[dom]["ms_per_launch"] * per_layer / 1e3
     xf, xb = kernel_work(dom, path, N, E, H, H, H, H, FE, g1, s)     # the layer's work
