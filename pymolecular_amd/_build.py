@@ -41,6 +41,7 @@ FILE_FLAGS = {
     "egnn_mpnn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "egnn_eqfwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "egnn_wfwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "egnn_wbwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "egnn_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "egnn_f32s.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }

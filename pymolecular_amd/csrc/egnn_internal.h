@@ -309,6 +309,13 @@ int launch_wide_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
 // The backward runs one persistent 16-wave block per CU and writes per-block partials of dw2_mov
 // and dw_d ([nblk][M | H], EGNN) to BwdArgs::dwpart.
 constexpr int kWideBwdBlocks = 256;
+// The edge-parallel kernel (egnn_wbwd.hip) takes a pass of the chip per 256 x 128 edges, about 38 us however few of its
+// waves have edges; the one that shares a 32-edge tile over eight waves a round per 256 tiles, about 10 + 12 us a round.
+// Measured, edge-parallel against shared: 2.7k edges 38 / 22 us, 10.8k 38 / 34, 30k 42 / 58, 61k 75 / 105, 122k 155 / 190,
+// 661k 815 / 990.
+inline bool wide_bwd_ep(int64_t E) { return 38 * cdiv(E, 256 * 128) < 10 + 12 * cdiv(E, 256 * kTileEdges); }
+int wide_bwd_ep_blocks(int64_t E);
+int launch_wide_bwd_ep(const LayerShape& s, const BwdArgs& a, int nblk, hipStream_t st);
 int wide_bwd_blocks(const LayerShape& s);
 int launch_wide_bwd(const LayerShape& s, const BwdArgs& a, int nblk, hipStream_t st);
 // fp32 edge kernels on split operands (egnn_f32.hip): H = O = M = 128

@@ -1,4 +1,5 @@
-// Workgroup-cooperative fused backward for wide layers (bf16, H = O = M = 256, gfx950); the forward is
+// Workgroup-cooperative fused backward for wide layers (bf16, H = O = M = 256, gfx950) of few edges (wide_bwd_ep):
+// with eight waves on one tile a small graph's edges reach every CU.  Larger graphs run egnn_wbwd.hip; the forward is
 // egnn_wfwd.hip.
 //
 // Same tile organisation as the H = 128 kernels: all W = 8 waves of a block
@@ -516,10 +517,13 @@ bool wide_supported(const LayerShape& s) {
 }
 
 int wide_bwd_blocks(const LayerShape& s) {
-  return (int)std::min<int64_t>(cdiv(std::max<int64_t>(s.E, 1), kTileEdges), kWideBwdBlocks);
+  const int64_t E = std::max<int64_t>(s.E, 1);
+  if (wide_bwd_ep(E)) return wide_bwd_ep_blocks(E);
+  return (int)std::min<int64_t>(cdiv(E, kTileEdges), kWideBwdBlocks);
 }
 
 int launch_wide_bwd(const LayerShape& s, const BwdArgs& a, int nblk, hipStream_t st) {
+  if (wide_bwd_ep(s.E)) return launch_wide_bwd_ep(s, a, nblk, st);
   if (s.eq)
     return s.NUC == 1 ? launch_wide_bwd_t<256, 8, true, 1>(a, nblk, st) : launch_wide_bwd_t<256, 8, true, 2>(a, nblk, st);
   return s.NUC == 1 ? launch_wide_bwd_t<256, 8, false, 1>(a, nblk, st) : launch_wide_bwd_t<256, 8, false, 2>(a, nblk, st);
