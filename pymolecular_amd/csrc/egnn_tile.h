@@ -89,15 +89,6 @@ __device__ __forceinline__ int rank_of(uint32_t mask, int k) {
   return __popc(mask & below) - 1;
 }
 
-// A operand that adds two 4-row halves of a B chunk: A[r][8g + s] = (r == 4g + (s & 3)), so
-// the product with B = [P rows 4g..4g+3 | Q rows 4g..4g+3] (lane g) is P + Q on rows 4g..4g+3
-__device__ __forceinline__ bf16x8 pair_sum_chunk(int c, int g) {
-  bf16x8 r;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) r[s] = (c - 4 * g == (s & 3)) ? (bf16)1.0f : (bf16)0.0f;
-  return r;
-}
-
 // P_i + Q_j of a 16-feature block from one gathered B chunk: lanes g = 0, 1 of
 // edge column c hold P features 8g .. 8g + 7 of the block, lanes g = 2, 3 Q
 // features 8(g - 2) .. + 7 (pq_gather); A[r][k] = 1 where k is P or Q feature r.

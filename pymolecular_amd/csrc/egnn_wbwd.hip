@@ -14,6 +14,8 @@
 // reads and barriers bound it.
 // Measured against the kernel that shares a 32-edge tile over eight waves by feature rows (661k edges, F_E = 32):
 // 990 -> 815 us; the weights' loads through generic pointers, whose waits join those of the LDS, cost 20 us of it.
+// Every stage sums in the order of egnn_wide.hip (biases, P_i and Q_j onto the finished products, g_m as the first term), so
+// the factors and Gh are bit for bit those of that kernel.
 // A lane past the last edge computes that edge again and stores the same values, so no store is under a branch.
 #include "egnn_device.h"
 #include "egnn_internal.h"
@@ -118,7 +120,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
   const int fsum = 16 * (c >> 2) + 4 * g + (c & 3);
   __syncthreads();
 
-  const bf16x8 Ipq = pair_sum_chunk(c, g);
   // the edge's row, source and edge id, one pass ahead (without edge ids a stand-in read, ignored)
   const int32_t* eidp = a.eids ? a.eids : a.erow;
   int n_ri, n_rj, n_eid;
@@ -171,9 +172,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int kc = k4 + k;
-        f32x4 y[2] = {zero4(), zero4()};
-        mma(y[0], Ipq, __builtin_shufflevector(p[k], q[k], 0, 1, 2, 3, 8, 9, 10, 11));
-        mma(y[1], Ipq, __builtin_shufflevector(p[k], q[k], 4, 5, 6, 7, 12, 13, 14, 15));
+        f32x4 y[2] = {zero4(), zero4()}, pv[2], qv[2];
+        unpack_chunk(p[k], pv[0], pv[1]);
+        unpack_chunk(q[k], qv[0], qv[1]);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
 #pragma unroll
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
           f32x4 d;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const YD r = silu_yd<bf16>(y[b][i]);
+            const YD r = silu_yd<bf16>(y[b][i] + pv[b][i] + qv[b][i]);
             y[b][i] = r.y;
             d[i] = r.d;
           }
@@ -197,16 +198,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
     bf16x4 s2[O / 16];
 #pragma unroll
     for (int k = 0; k < O / 32; ++k) {   // 32 rows at a time, chunk k / 2
-      f32x4 acc[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) acc[b] = *reinterpret_cast<const f32x4*>(s_vec + 32 * k + 16 * b + 4 * g);
+      f32x4 acc[2] = {zero4(), zero4()};
       rows(k >> 1, k & 1, m1, acc);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
+        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * k + 16 * b + 4 * g);
         f32x4 d;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd<bf16>(acc[b][i]);
+          const YD r = silu_yd<bf16>(acc[b][i] + b2[i]);
           acc[b][i] = r.y;
           d[i] = r.d;
         }
@@ -231,9 +231,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
       float pv[16];
 #pragma unroll
       for (int k = 0; k < M / 32; ++k) {
-        f32x4 acc[2];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[b] = *reinterpret_cast<const f32x4*>(s_vec + O + 32 * k + 16 * b + 4 * g);
+        f32x4 acc[2] = {zero4(), zero4()};
         if (k + 1 == M / 32) {
           gr0 = *reinterpret_cast<const bf16x4*>(gm);
           gr1 = *reinterpret_cast<const bf16x4*>(gm + 16);
@@ -241,10 +239,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
         rows(kST + (k >> 1), k & 1, mc, acc);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
+          const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 32 * k + 16 * b + 4 * g);
           const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 32 * k + 16 * b + 4 * g);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const YD r = silu_yd<bf16>(acc[b][i]);
+            const YD r = silu_yd<bf16>(acc[b][i] + bx[i]);
             phi += r.y * w2[i];
             pv[8 * (k & 1) + 4 * b + i] = gpm * r.y;
             acc[b][i] = gphi * w2[i] * r.d;
@@ -269,10 +268,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) 
         gr0 = *reinterpret_cast<const bf16x4*>(gm + 32 * (k + 1));
         gr1 = *reinterpret_cast<const bf16x4*>(gm + 32 * (k + 1) + 16);
       }
-      f32x4 acc[2] = {zero4(), zero4()};
+      f32x4 acc[2] = {unpack4(g0), unpack4(g1)};
       if constexpr (EQ) rows(2 * kST + (k >> 1), k & 1, gq, acc);
-      acc[0] += unpack4(g0);
-      acc[1] += unpack4(g1);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         acc[b] *= unpack4(s2[2 * k + b]);

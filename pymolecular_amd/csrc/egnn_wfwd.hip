@@ -2,9 +2,12 @@
 //
 // Each wave takes whole 32-edge schedule tiles and runs both 16-edge halves side by side in its own registers with the
 // features on the MFMA rows, so every weight fragment read from LDS feeds two products:
-//   S1  m1 = SiLU(W_u [e | r^2] + P_i + Q_j)    (the P_i + Q_j sum an MFMA against a 0/1 operand)
+//   S1  m1 = SiLU(W_u [e | r^2] + P_i + Q_j)
 //   S2  m  = SiLU(W_hl^T m1 + b2), 32 rows at a time; their row sums right away
 //   S3  phi = SiLU(W1_mov^T m + bx1) . w2_mov, 32 rows at a time
+// P_i, Q_j and the biases are added to the finished products in fp32, in the order of egnn_wide.hip, so the messages are
+// bit for bit those of the tile-sharing kernels (a P_i + Q_j by a product against a 0/1 operand saves 500 vector
+// instructions a pass, but rounds differently and turns an infinite feature into 16 NaNs).
 // The two 256 x 256 weights (256 KB) do not fit the LDS: 16 KB chunks of 32 rows go through two LDS buffers in the
 // order of use, shared by the block's four waves, the next chunk loaded into registers before the products of the
 // current one and stored after them, one barrier per chunk.  W_u's fragments stay in LDS.  75 KB leave two blocks per
@@ -27,7 +30,7 @@ constexpr int kChunkElems = 2 * KH * kFragElems;   // 32 rows
 
 template <bool EQ, int NU>   // NU: 32-slot slices of the edge input (1 or 2)
 __global__ __launch_bounds__(64 * kWaves, 2) void wide_fwd_ep_kernel(FwdArgs a) {
-  constexpr int SEGW = O + (EQ ? 4 : 0), NCH = EQ ? 2 * KP : KP;
+  constexpr int SEGW = O + (EQ ? 4 : 0), NCH = EQ ? 2 * KP : KP, KG = 4;
   __shared__ __attribute__((aligned(16))) bf16 s_w[2][kChunkElems];
   __shared__ __attribute__((aligned(16))) bf16 s_u[2 * KH * NU * kFragElems];
   __shared__ __attribute__((aligned(16))) float s_vec[O + 2 * M];             // b2 | bx1 | w2_mov
@@ -96,7 +99,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_fwd_ep_kernel(FwdArgs a) 
   stream_store(0);
   __syncthreads();
 
-  const bf16x8 Ipq = pair_sum_chunk(c, g);
   for (int64_t ps = blockIdx.x; ps < npass; ps += gridDim.x) {
     __asm__ __volatile__("" : "+v"(so));
     const int64_t T0 = ps * kWaves + w;
@@ -133,33 +135,39 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_fwd_ep_kernel(FwdArgs a) 
     // ---- S1
     bf16x8 m1[KH][2];
 #pragma unroll
-    for (int k4 = 0; k4 < KH; k4 += 4) {
-      bf16x8 p[4][2], q[4][2];
+    for (int k4 = 0; k4 < KH; k4 += KG) {
+      bf16x8 p[KG][2], q[KG][2];
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < KG; ++k)
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
           p[k][nb] = load_chunk(PQ + (int64_t)ri[nb] * 2 * H + 32 * (k4 + k) + 8 * g);
           q[k][nb] = load_chunk(PQ + (int64_t)rj[nb] * 2 * H + H + 32 * (k4 + k) + 8 * g);
         }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < KG; ++k) {
         const int kc = k4 + k;
         f32x4 y[2][2];   // [row block][edge block]
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          y[0][nb] = y[1][nb] = zero4();
-          mma(y[0][nb], Ipq, __builtin_shufflevector(p[k][nb], q[k][nb], 0, 1, 2, 3, 8, 9, 10, 11));
-          mma(y[1][nb], Ipq, __builtin_shufflevector(p[k][nb], q[k][nb], 4, 5, 6, 7, 12, 13, 14, 15));
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 2; ++b) {
+          y[b][0] = y[b][1] = zero4();
 #pragma unroll
           for (int uc = 0; uc < NU; ++uc) {
             const bf16x8 A = load_chunk(s_u + (((2 * kc + b) * NU + uc) * 64 + l) * 8);
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) mma(y[b][nb], A, u[uc][nb]);
           }
+        }
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+          f32x4 pv[2], qv[2];
+          unpack_chunk(p[k][nb], pv[0], pv[1]);
+          unpack_chunk(q[k][nb], qv[0], qv[1]);
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[b][nb][i] = y[b][nb][i] + pv[b][i] + qv[b][i];
+        }
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
@@ -174,16 +182,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_fwd_ep_kernel(FwdArgs a) 
     bf16x8 mc[EQ ? KP : 1][2];
 #pragma unroll
     for (int kp = 0; kp < KP; ++kp) {
-      f32x4 acc[2][2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) acc[b][0] = acc[b][1] = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
+      f32x4 acc[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
       rows(kp, m1, acc);
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < 2; ++b) {
+          const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[b][nb][i] = silu_t<bf16>(acc[b][nb][i]);
+          for (int i = 0; i < 4; ++i) acc[b][nb][i] = silu_t<bf16>(acc[b][nb][i] + b2[i]);
+        }
         const bf16x8 v = pack_chunk<bf16>(acc[0][nb], acc[1][nb]);
         if constexpr (EQ) mc[kp][nb] = v;
         store_chunk(s_msg[w] + (nb * 64 + chain_slot<true>(l)) * 8, v);
@@ -215,18 +223,18 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_fwd_ep_kernel(FwdArgs a) 
       float phi[2] = {0.f, 0.f};
 #pragma unroll
       for (int mp = 0; mp < M / 32; ++mp) {
-        f32x4 acc[2][2];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[b][0] = acc[b][1] = *reinterpret_cast<const f32x4*>(s_vec + O + 32 * mp + 16 * b + 4 * g);
+        f32x4 acc[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
         rows(KP + mp, mc, acc);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
+          const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 32 * mp + 16 * b + 4 * g);
           const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 32 * mp + 16 * b + 4 * g);
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) phi[nb] += silu_t<bf16>(acc[b][nb][i]) * w2[i];
+            for (int i = 0; i < 4; ++i) phi[nb] += silu_t<bf16>(acc[b][nb][i] + bx[i]) * w2[i];
         }
+        __asm__ __volatile__("" : "+v"(phi[0]), "+v"(phi[1]));   // summed here: else the eight steps' sums are kept to the end
         __syncthreads();
       }
 #pragma unroll

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from tests.cases import Case, random_csr
-from tests.test_fused_gpu import check_case
+from tests.test_fused_gpu import check_case, run_fused
 
 pytestmark = pytest.mark.gpu
 
@@ -27,3 +27,24 @@ def test_many_passes(E, eq):
     degs = [33] * (E // 33) + [E % 33]
     rowptr, col = random_csr(len(degs), degs, seed=7)
     check_case(Case(rowptr, col, 16, 16, 256, 256, 256, seed=62, eq=eq), "bf16")
+
+
+@pytest.mark.parametrize("eq,fe", [(True, 32), (True, 56), (False, 8)])
+def test_same_bits_on_both_sides_of_the_rule(eq, fe):
+    """A graph of 8,192 edges (the kernel that shares a tile) alone and as the first part of one of 17,600 (the
+    edge-parallel kernel): the gradient of its nodes' features is the same to the bit, as every stage of the two kernels
+    sums in the same order."""
+    part, rest = [32] * 256, [40] * 235 + [8, 0]
+    rowptr, col = random_csr(256, part, seed=9)
+    more, col2 = random_csr(len(rest), rest, seed=10)
+    whole = Case(np.concatenate([rowptr, rowptr[-1] + more[1:]]), np.concatenate([col, 256 + col2]), 64, fe, 256, 256, 256,
+                 seed=63, eq=eq, mean_agg=eq)
+    alone = Case(rowptr, col, 64, fe, 256, 256, 256, seed=63, eq=eq, mean_agg=eq)
+    alone.p = whole.p
+    n = alone.N
+    alone.h, alone.gm, alone.ef = whole.h[:n], whole.gm[:n], whole.ef[:alone.E]
+    if eq:
+        alone.coord, alone.gx = whole.coord[:n], whole.gx[:n]
+    a, b = run_fused(alone, "bf16"), run_fused(whole, "bf16")
+    assert np.array_equal(a["out_msg"], b["out_msg"][:n])
+    assert np.array_equal(a["grads"]["h"], b["grads"]["h"][:n])

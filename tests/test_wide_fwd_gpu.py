@@ -4,7 +4,7 @@ import pytest
 
 from tests.cases import Case, random_csr
 from tests.test_f32_split_gpu import _degrees
-from tests.test_fused_gpu import check_case
+from tests.test_fused_gpu import check_case, run_fused
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +32,15 @@ def test_many_passes():
     degs = np.full(2100, 33)
     rowptr, col = random_csr(len(degs), degs, seed=6)
     check_case(Case(rowptr, col, 16, 16, 256, 256, 256, seed=53, bias=False), "bf16", backward=False)
+
+
+@pytest.mark.parametrize("eq", [True, False])
+def test_infinite_feature(eq):
+    """One infinite entry of b1: an infinite message where its weight is positive, SiLU(-inf) = NaN where it is negative,
+    as in the oracle (rows of 32 edges, so that no row sum multiplies another row's infinity by 0)."""
+    rowptr, col = random_csr(40, np.full(40, 32), seed=8)
+    case = Case(rowptr, col, 32, 8, 256, 256, 256, seed=54, eq=eq)
+    case.p["b1"][37] = np.inf
+    got = run_fused(case, "bf16", backward=False)["out_msg"]
+    up = case.p["w2_msg"][37] > 0
+    assert np.isposinf(got[:, up]).all() and np.isnan(got[:, ~up]).all()
