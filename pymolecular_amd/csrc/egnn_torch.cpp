@@ -29,9 +29,10 @@ void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device
 template <typename T = void> T* ptr(const Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
 Tensor get(const Opt& t) { return t.has_value() ? *t : Tensor(); }
 bool aligned16(const Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
-// unit-stride rows that start 16-byte aligned, else a contiguous copy
+// unit-stride rows that start 16-byte aligned and do not overlap (an expanded gradient's have stride 0), else a copy
 Tensor rowmajor(const Tensor& t) {
-  return t.stride(1) == 1 && (t.stride(0) * t.element_size()) % 16 == 0 && aligned16(t) ? t : t.contiguous();
+  return t.stride(1) == 1 && t.stride(0) >= t.size(1) && (t.stride(0) * t.element_size()) % 16 == 0 && aligned16(t)
+             ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
 // no tensor subclass, functorch wrapper or functionalised tensor, on h's device

@@ -203,6 +203,15 @@ def _as(t: Optional[torch.Tensor], dt: torch.dtype) -> Optional[torch.Tensor]:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def _rowmajor(t: torch.Tensor) -> torch.Tensor:
+    """``t`` if its rows are unit-stride, 16-byte aligned and apart, else a contiguous copy.  (A sum over the
+    nodes sends one row expanded with stride 0; a contiguous tensor may start at an unaligned offset.)"""
+    esz = t.element_size()
+    if t.stride(1) == 1 and t.stride(0) >= t.shape[1] and (t.stride(0) * esz) % 16 == 0 and t.data_ptr() % 16 == 0:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
 def _prep_inputs(h, coord, edge_feat, w1, w2, w1m, w2m, b1, b2, bx1, equivariant):
     _require_device(h, "h")
     dt = h.dtype
@@ -327,9 +336,7 @@ def _fused_backward(h, coord, edge_feat, row_ptrs, col_indices, edge_ids, w1, w2
         sched = get_schedule(row_ptrs, col_indices, h.shape[0])
     dev, dt = h.device, h.dtype
     N = h.shape[0]
-    gm = grad_out_msg.to(dt)
-    if gm.stride(1) != 1 or (gm.stride(0) * gm.element_size()) % 16 or gm.data_ptr() % 16:
-        gm = gm.contiguous()   # the kernels read 8- and 16-byte pieces of unit-stride rows
+    gm = _rowmajor(grad_out_msg.to(dt))   # the kernels read 8- and 16-byte pieces of unit-stride rows
     gx = _as(grad_out_mov, torch.float32) if equivariant else None
     if grad_h_into is not None:
         gh = grad_h_into

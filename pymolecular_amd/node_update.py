@@ -17,17 +17,9 @@ import torch
 
 from . import _capi
 from ._capi import EgnnNodeDims, check
-from .fused import _as, _stream
+from .fused import _as, _rowmajor, _stream
 
 __all__ = ["NodeUpdateFn", "node_update", "node_update_forward", "node_update_backward", "DenseFn", "dense"]
-
-
-def _rowmajor(t: torch.Tensor) -> torch.Tensor:
-    """``t`` if its rows are unit-stride with 16-byte aligned row starts, else a contiguous copy."""
-    esz = t.element_size()
-    if t.stride(1) == 1 and (t.stride(0) * esz) % 16 == 0 and t.data_ptr() % 16 == 0:
-        return t
-    return t.contiguous()
 
 
 def _dims(x1, x2, w1, w2, residual) -> EgnnNodeDims:
