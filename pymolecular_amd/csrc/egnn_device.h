@@ -135,6 +135,24 @@ __device__ __forceinline__ float shfl_xor(float v, int m) { return __shfl_xor(v,
 __device__ __forceinline__ float shfl(float v, int src) { return __shfl(v, src, 64); }
 __device__ __forceinline__ int shfl_i(int v, int src) { return __shfl(v, src, 64); }
 
+// v[j] and v[j + N] of two lanes -> the sum of one of them in each: N values left
+template <int DPP, int N>
+__device__ __forceinline__ void halve(float* v, bool up) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float keep = up ? v[j + N] : v[j], send = up ? v[j] : v[j + N];
+    v[j] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), DPP, 0xf, 0xf, false));
+  }
+}
+// 16 values a lane, summed over the 16 edges (lanes c): lane c keeps value c
+__device__ __forceinline__ float edge_sum16(float* v, int c) {
+  halve<0x128, 8>(v, c & 8);   // row_ror:8
+  halve<0x141, 4>(v, c & 4);   // row_half_mirror
+  halve<0x4E, 2>(v, c & 2);    // quad_perm [2, 3, 0, 1]
+  halve<0xB1, 1>(v, c & 1);    // quad_perm [1, 0, 3, 2]
+  return v[0];
+}
+
 // an index forced into [0, n) (n >= 1): out-of-range values, negative ones included, become n - 1
 __device__ __forceinline__ int clampi(int v, int n) { return (int)__builtin_elementwise_min((unsigned)v, (unsigned)(n - 1)); }
 

@@ -63,6 +63,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, g = l >> 4;
   const int h = w & 1, pr = w >> 1;
+  const float sg = c & 1 ? -1.0f : 1.0f;   // the edge's sign in the chain
   const float* PQ = (const float*)a.PQ;
   const float* ef = (const float*)a.ef;
   const int64_t E = a.E;
@@ -139,13 +140,13 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
           f32x8 u = zero_chunk<float>();
           if (s0 + 8 <= a.FE) u = load_chunk(ef + (int64_t)eid * a.se + s0);
           else if (EQ && s0 == a.FE) u.lo[0] = r2;
-          const Chunk3 u3 = split_chunk(u.lo, u.hi);
+          const Chunk3 u3 = split_chunk(u.lo * sg, u.hi * sg);
 #pragma unroll
           for (int rb = 0; rb < H / 16; ++rb) {
             const Chunk3 A = lds_chunk3((const bf16*)a.fr.s_u + ((int64_t)(rb >> 1) * 6 * a.NUC + ((rb & 1) * a.NUC + uc) * 3) * kFragElems, l);
             f32x4 lo = zero4(), hi = zero4();
             mma3(hi, lo, A, u3);
-            y[rb >> 1][rb & 1] += hi + lo;
+            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], hi + lo, sg);
           }
         }
       } else if constexpr (EQ) {
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) y[kc][b][i] = silu_f32(y[kc][b][i]);
+          for (int i = 0; i < 4; ++i) y[kc][b][i] = silu_f32(y[kc][b][i], sg);
         m1[kc] = split_chunk(y[kc][0], y[kc][1]);
       }
     }
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
         for (int b = 0; b < 2; ++b) {
           const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) x[b][i] = silu_f32(hi[b][i] + (lo[b][i] + b2[i]));
+          for (int i = 0; i < 4; ++i) x[b][i] = silu_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
           *reinterpret_cast<f32x4*>(mrow + c * SP + 32 * (kp & 1) + 16 * b + 4 * g) = x[b];
         }
         stream_store((CH * kp + 1) & 1);
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
         bool deferred = h && cont;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
-          acc += v[k];
+          acc += k & 1 ? -v[k] : v[k];   // the rows hold the signed messages
           if ((mine >> k) & 1u) {
             if (deferred) {
               first[kp >> 1] = acc;
@@ -264,7 +265,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
         const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 16 * rb + 4 * g);
         const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * rb + 4 * g);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) phi += silu_f32(q[rb][i] + bx[i]) * w2[i];
+        for (int i = 0; i < 4; ++i) phi += silu_f32(__builtin_fmaf(q[rb][i], sg, bx[i])) * w2[i];
       }
       phi += shfl_xor(phi, 16);
       phi += shfl_xor(phi, 32);
@@ -308,35 +309,12 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
   }
 }
 
-// Sums over the 16 edges (lanes c) of 32 per-lane values, scattered: lane c of a 16-lane row ends with the sums
-// of values 2 c and 2 c + 1.  Four exchange steps, each halving the values a lane keeps; the partners differ in
-// bit 3, 2, 1, 0 of c.
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL, int N>
-__device__ __forceinline__ void scatter_step(float* v, bool up) {
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const float keep = up ? v[k + N] : v[k], send = up ? v[k] : v[k + N];
-    v[k] = keep + dpp<CTRL>(send);
-  }
-}
-__device__ __forceinline__ f32x2 edge_sums(float* v, int c) {
-  scatter_step<0x128, 16>(v, c & 8);   // row_ror:8
-  scatter_step<0x141, 8>(v, c & 4);    // row_half_mirror
-  scatter_step<0x4E, 4>(v, c & 2);     // quad_perm [2, 3, 0, 1]
-  scatter_step<0xB1, 2>(v, c & 1);     // quad_perm [1, 0, 3, 2]
-  return f32x2{v[0], v[1]};
-}
-
 // Backward over 16 edges per wave, the chain of egnn_bwd.hip with every product on split operands:
 //   S1 m1, SiLU'   S2 m, SiLU' (32 rows at a time)   S3 q += W1_mov^T m over those rows
 //   g_q = g_phi w2_mov SiLU'(q)   S4 g_m = gm_i + W1_mov g_q, g_a2 = g_m SiLU' (32 rows at a time)
 //   S5 g_a1 += W_hl g_a2 over those rows   S6 dL/ddelta = phi gx_i + 2 (w_d . g_a1) delta
 // The weights go through LDS as in the forward, 16 chunks a pass.  Stores Gh, Gx and the factors m1, m, g_q, g_a2
-// for atb_f32_kernel; dw2_mov = sum g_phi p and dw_d = sum r^2 g_a1 are summed here (edge_sums over the wave's
+// for atb_f32_kernel, all four with the edge's sign (odd edges negative: the products are the same); dw2_mov = sum g_phi p and dw_d = sum r^2 g_a1 are summed here (edge_sum16 over the wave's
 // edges, then registers over the passes) into one partial row [M | H] per block.
 // Measured against one wave per 32-edge tile on the fp32 instruction, which also stored p and r^2 for dw2_mov and
 // dw_d: 989 -> 527 us at 394k edges, 146 -> 90 us at 46k (both in two chunks).
@@ -352,6 +330,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
   static_assert(sizeof(float) * kF32Waves * (M + H) <= sizeof(s_w[0]), "the final sums reuse the weight buffer");
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+  const float sg = c & 1 ? -1.0f : 1.0f;   // the edge's sign in the chain
   const float* PQ = (const float*)a.PQ;
   const float* ef = (const float*)a.ef;
   const float* gmsg = (const float*)a.gmsg;
@@ -429,7 +408,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
   stream_store(0, 0);
   stream_load(0, 1);
   stream_store(0, 1);
-  f32x2 sw2 = {0.f, 0.f}, swd = {0.f, 0.f};   // the lane's sums of dw2_mov and dw_d (features of edge_sums)
+  float sw2[2] = {0.f, 0.f}, swd[2] = {0.f, 0.f};   // the lane's sums of dw2_mov and dw_d: feature fsum of each 64
+  const int fsum = 16 * (c >> 2) + 4 * g + (c & 3);
   __syncthreads();
 
   for (int64_t ps = blockIdx.x; ps < npass; ps += gridDim.x) {
@@ -479,13 +459,13 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
           f32x8 u = zero_chunk<float>();
           if (s0 + 8 <= a.FE) u = load_chunk(ef + (int64_t)eid * a.se + s0);
           else if (EQ && s0 == a.FE) u.lo[0] = r2;
-          const Chunk3 u3 = split_chunk(u.lo, u.hi);
+          const Chunk3 u3 = split_chunk(u.lo * sg, u.hi * sg);
 #pragma unroll
           for (int rb = 0; rb < H / 16; ++rb) {
             const Chunk3 A = lds_chunk3((const bf16*)a.fr.s_u + ((int64_t)(rb >> 1) * 6 * a.NUC + ((rb & 1) * a.NUC + uc) * 3) * kFragElems, l);
             f32x4 lo = zero4(), hi = zero4();
             mma3(hi, lo, A, u3);
-            y[rb >> 1][rb & 1] += hi + lo;
+            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], hi + lo, sg);
           }
         }
       } else if constexpr (EQ) {
@@ -503,7 +483,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
           f32x4 d;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const YD r = silu_yd_f32(y[kc][b][i]);
+            const YD r = silu_yd_f32(y[kc][b][i], sg);
             y[kc][b][i] = r.y;
             d[i] = r.d;
           }
@@ -530,7 +510,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
         const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(hi[b][i] + (lo[b][i] + b2[i]));
+          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
           x[b][i] = r.y;
           s2[kp][b][i] = r.d;
         }
@@ -542,7 +522,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
     float phi = 0.f;
     Chunk3 gq[EQ ? M / 32 : 1];
     if constexpr (EQ) {
-      float pv[M / 4];
+      float pv[16];
+      const float gpsg = gphi * sg;
 #pragma unroll
       for (int kc = 0; kc < M / 32; ++kc) {
 #pragma unroll
@@ -552,18 +533,20 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
           const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * rb + 4 * g);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const YD r = silu_yd_f32(q[rb][i] + bx[i]);
+            const YD r = silu_yd_f32(__builtin_fmaf(q[rb][i], sg, bx[i]), sg);
             phi += r.y * w2[i];
-            pv[4 * rb + i] = gphi * r.y;
+            pv[4 * (rb & 3) + i] = gpsg * r.y;
             q[rb][i] = gphi * w2[i] * r.d;
           }
           if (valid) *reinterpret_cast<f32x4*>((float*)a.Dgq + fo + 16 * rb) = q[rb];
         }
         gq[kc] = split_chunk(q[2 * kc], q[2 * kc + 1]);
+        if (kc & 1) sw2[kc >> 1] += edge_sum16(pv, c);
+        __asm__ __volatile__("" : "+v"(phi));   // summed here, not at the end of all four
       }
+      phi *= sg;
       phi += shfl_xor(phi, 16);
       phi += shfl_xor(phi, 32);
-      sw2 += edge_sums(pv, c);
     }
     // ---- S4, S5
     f32x4 ga1[H / 16];
@@ -580,7 +563,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
         f32x4 hi[2] = {zero4(), zero4()}, lo[2] = {zero4(), zero4()};
         rows_chunk(2 * KP + 2 * kp, gq, hi, lo);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) x[b] += hi[b] + lo[b];
+        for (int b = 0; b < 2; ++b) x[b] = add_signed(x[b], hi[b] + lo[b], sg);
       }
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
@@ -591,7 +574,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
     }
     // ---- Gh, S6, dw_d
     {
-      float gr = 0.f, gv[H / 4];
+      float gr = 0.f, gv[16];
       const int64_t go = (ee - a.gbase) * H + 4 * g;
 #pragma unroll
       for (int rb = 0; rb < H / 16; ++rb) {
@@ -602,8 +585,10 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             gr += v[i] * wd[i];
-            gv[4 * rb + i] = r2 * v[i];
+            gv[4 * (rb & 3) + i] = r2 * v[i];
           }
+          if ((rb & 3) == 3) swd[rb >> 2] += edge_sum16(gv, c);
+          __asm__ __volatile__("" : "+v"(gr));
         }
       }
       if constexpr (EQ) {
@@ -614,17 +599,16 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
           *reinterpret_cast<f32x4*>(a.Gx + (ee - a.gbase) * 4) =
               f32x4{phi * gxx + k2 * dx, phi * gxy + k2 * dy, phi * gxz + k2 * dz, gphi};
         }
-        swd += edge_sums(gv, c);
       }
     }
   }
   if constexpr (EQ) {   // the block's partial row: the waves' sums in wave order, added to an earlier chunk's
-    const int f = 16 * (c >> 1) + 4 * g + 2 * (c & 1);   // the features of values 2 c, 2 c + 1
     float* const s_sum = (float*)s_w[0];   // [wave][M | H]; the passes ended with a barrier
-    s_sum[w * (M + H) + f] = sw2[0];
-    s_sum[w * (M + H) + f + 1] = sw2[1];
-    s_sum[w * (M + H) + M + f] = swd[0];
-    s_sum[w * (M + H) + M + f + 1] = swd[1];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s_sum[w * (M + H) + 64 * h + fsum] = sw2[h];
+      s_sum[w * (M + H) + M + 64 * h + fsum] = swd[h];
+    }
     __syncthreads();
     float* row = a.dwpart + (int64_t)blockIdx.x * (M + H);
     for (int q = threadIdx.x; q < M + H; q += 64 * kF32Waves) {
@@ -641,7 +625,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
 // (eight waves, one per CU) computes the whole 128 x 128 result of its range: slices of 32 edges, split into
 // parts on the way to LDS ([edge][column] rows of 288 bytes, which the transposing reads of 32 lanes cross
 // without bank conflicts), two slices in flight in registers and two in LDS.  The ones row (bias gradient) is the
-// sum of the B values each thread loads, in fp32.  Each block adds to its partial row of an earlier chunk.
+// sum of the B values each thread loads, in fp32, odd edges subtracted (their rows are stored negative).  Each block adds to its partial row of an earlier chunk.
 // Measured (both products, two chunks, with the matrix-vector products the backward kernel now sums itself):
 // 750 -> 222 us at 394k edges (3.6 TB/s), 123 -> 41 us at 46k.
 constexpr int kAtbPitch = 144, kAtbSlice = 32, kAtbThreads = 512;
@@ -656,7 +640,7 @@ __global__ __launch_bounds__(kAtbThreads, 2) void atb_f32_kernel(AtbF32Args a) {
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15, g = l >> 4;
   const float* A = blockIdx.y ? a.A1 : a.A0;
   const float* B = blockIdx.y ? a.B1 : a.B0;
-  const int64_t kb = (int64_t)blockIdx.x * a.len;
+  const int64_t kb = (int64_t)blockIdx.x * a.len;   // len: a multiple of 64
   const int64_t ke = kb + a.len < a.K ? kb + a.len : a.K;
   const uint32_t flip = (blockIdx.x & 1) << 31;   // every other range (flip_sign)
   const float sgn = flip ? -1.0f : 1.0f;
@@ -736,7 +720,7 @@ __global__ __launch_bounds__(kAtbThreads, 2) void atb_f32_kernel(AtbF32Args a) {
         *o = a.add ? *o + v : v;
       }
   float* s = (float*)s_ab;   // [16][128] sums of the thread rows
-  *reinterpret_cast<f32x4*>(s + row * 128 + q4) = ones;
+  *reinterpret_cast<f32x4*>(s + row * 128 + q4) = row & 1 ? -ones : ones;
   __syncthreads();
   if (tid < 128) {
     float v = 0.f;

@@ -71,6 +71,7 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
   __shared__ __attribute__((aligned(16))) float s_msg[kW][kTileEdges * SP];
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+  const float sg = c & 1 ? -1.0f : 1.0f;   // the edge's sign in the chain
   const float* PQ = (const float*)a.PQ;
   const float* ef = (const float*)a.ef;
   const int64_t E = a.E;
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
       Chunk3 u3[2];
       if constexpr (U) {
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) u3[nb] = split_chunk(u[nb].lo, u[nb].hi);
+        for (int nb = 0; nb < 2; ++nb) u3[nb] = split_chunk(u[nb].lo * sg, u[nb].hi * sg);
       }
 #pragma unroll
       for (int rb = 0; rb < H / 16; ++rb) {
@@ -132,12 +133,12 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb) mma3(hi[nb], lo[nb], A, u3[nb]);
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb) y[rb >> 1][nb][rb & 1] += hi[nb] + lo[nb];
+          for (int nb = 0; nb < 2; ++nb) y[rb >> 1][nb][rb & 1] = add_signed(y[rb >> 1][nb][rb & 1], hi[nb] + lo[nb], sg);
         }
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) y[rb >> 1][nb][rb & 1][i] = silu_f32(y[rb >> 1][nb][rb & 1][i]);
+          for (int i = 0; i < 4; ++i) y[rb >> 1][nb][rb & 1][i] = silu_f32(y[rb >> 1][nb][rb & 1][i], sg);
         if (rb & 1) {
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb) m1[rb >> 1][nb] = split_chunk(y[rb >> 1][nb][0], y[rb >> 1][nb][1]);
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[nb][b][i] = silu_f32(hi[nb][i] + (lo[nb][i] + b2[i]));
+        for (int i = 0; i < 4; ++i) x[nb][b][i] = silu_f32(__builtin_fmaf(hi[nb][i] + lo[nb][i], sg, b2[i]), sg);
         *reinterpret_cast<f32x4*>(msg + (16 * nb + c) * SP + 16 * b + 4 * g) = x[nb][b];
       }
     }
@@ -180,10 +181,11 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) phi[nb] += silu_f32(hi[nb][i] + (lo[nb][i] + bx[i])) * w2[i];
+          for (int i = 0; i < 4; ++i) phi[nb] += silu_f32(__builtin_fmaf(hi[nb][i] + lo[nb][i], sg, bx[i])) * w2[i];
       }
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
+        phi[nb] *= sg;   // signed as the messages are
         phi[nb] += shfl_xor(phi[nb], 16);
         phi[nb] += shfl_xor(phi[nb], 32);
         if (g == 0)
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
         for (int k = 0; k < 8; ++k) v[k] = msg[(k0 + k) * SP + col];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-          acc += v[k];
+          acc += k & 1 ? -v[k] : v[k];   // the rows hold signed values
           ++n;
           if ((ends >> (k0 + k)) & 1u) {
             typedef __attribute__((address_space(1))) float gfloat;
@@ -319,7 +321,8 @@ __device__ __forceinline__ void mma3e(f32x4& acc0, f32x4& acc1, const Quad3& a, 
   mma16(acc1, a.p0, d.p0);
 }
 
-// sums over the 16 edges (lanes c) of eight values; lane c ends with that of value c >> 1
+// sums over the 16 edges (lanes c) of eight values that carry the edges' signs (odd lanes negative, so the exchanges with
+// a lane of the other parity subtract); lane c ends with that of value c >> 1, odd lanes with its negative
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
@@ -328,14 +331,15 @@ __device__ __forceinline__ float edge_sums8(const f32x4& a, const f32x4& b, int 
   f32x4 v;
 #pragma unroll
   for (int k = 0; k < 4; ++k) v[k] = (c & 8 ? b[k] : a[k]) + dpp<0x128>(c & 8 ? a[k] : b[k]);       // row_ror:8
-  const float p = (c & 4 ? v[2] : v[0]) + dpp<0x141>(c & 4 ? v[0] : v[2]);                           // row_half_mirror
-  const float q = (c & 4 ? v[3] : v[1]) + dpp<0x141>(c & 4 ? v[1] : v[3]);
+  const float p = (c & 4 ? v[2] : v[0]) - dpp<0x141>(c & 4 ? v[0] : v[2]);                           // row_half_mirror
+  const float q = (c & 4 ? v[3] : v[1]) - dpp<0x141>(c & 4 ? v[1] : v[3]);
   const float r = (c & 2 ? q : p) + dpp<0x4E>(c & 2 ? p : q);                                        // quad_perm [2, 3, 0, 1]
-  return r + dpp<0xB1>(r);                                                                           // quad_perm [1, 0, 3, 2]
+  return r - dpp<0xB1>(r);                                                                           // quad_perm [1, 0, 3, 2]
 }
 
 // The whole backward of 16 edges per wave: the chain of egnn_bwd.hip, then every weight gradient from the wave's own
-// operands, so nothing but Gh and Gx goes to memory.  The contractions over the edges (16-deep products) read both
+// operands, so nothing but Gh and Gx goes to memory.  m1, m, g_q, g_a2 and the edge inputs carry the edge's
+// sign, Gh does not; a product of two signed operands is what it was.  The contractions over the edges (16-deep products) read both
 // operands edge-major by transposing reads of the wave's 12 KB exchange buffer (m1, then g_a1; m, then g_a2; g_q,
 // then the edge inputs) and accumulate in 80 registers over the wave's edges; 32 edges at a time would use the
 // 32-deep products but not fit the registers.  The block's waves are added in wave order into one partial row in the
@@ -350,6 +354,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 s_x[kW][4 * kSlot];
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+  const float sg = c & 1 ? -1.0f : 1.0f;   // the edge's sign in the chain
   const float* PQ = (const float*)a.PQ;
   const float* ef = (const float*)a.ef;
   const float* gmsg = (const float*)a.gmsg;
@@ -406,7 +411,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
     f32x8 u;
     if constexpr (U) {
       const int eid = FEAT ? (a.eids ? clampi(a.eids[ee], (int)E) : (int)ee) : 0;
-      u = edge_slots<EQ, FEAT>(ef, a.se, eid, a.FE, g, d.r2);
+      u = edge_slots<EQ, FEAT>(ef, a.se, eid, a.FE, g, FEAT ? d.r2 : sg * d.r2);
     }
     // ---- S1
     f32x4 s1[4];
@@ -421,13 +426,18 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         y[2 * kc + 1] = p.hi + q.hi;
       }
       if constexpr (U) {
+        if constexpr (FEAT) {
+          const uint32_t odd = c & 1 ? 1u << 31 : 0u;
+          u.lo = flip_sign(u.lo, odd);
+          u.hi = flip_sign(u.hi, odd);
+        }
         const Chunk3 u3 = split_chunk(u.lo, u.hi);
 #pragma unroll
         for (int rb = 0; rb < 4; rb += 2) {
           f32x4 hi[2] = {zero4(), zero4()}, lo[2] = {zero4(), zero4()};
           mma3x2(hi, lo, frag3(s_u + rb * 3 * kFragElems, l), frag3(s_u + (rb + 1) * 3 * kFragElems, l), u3);
-          y[rb] += hi[0] + lo[0];
-          y[rb + 1] += hi[1] + lo[1];
+          y[rb] = add_signed(y[rb], hi[0] + lo[0], sg);
+          y[rb + 1] = add_signed(y[rb + 1], hi[1] + lo[1], sg);
         }
         opaque(u.lo);   // split again for d[W_e | w_d]
         opaque(u.hi);
@@ -436,7 +446,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(y[rb][i]);
+          const YD r = silu_yd_f32(y[rb][i], sg);
           y[rb][i] = r.y;
           s1[rb][i] = r.d;
         }
@@ -458,7 +468,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 16 * b + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(hi[b][i] + (lo[b][i] + b2[i]));
+          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
           x[b][i] = r.y;
           s2[b][i] = r.d;
         }
@@ -479,7 +489,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(hi[b][i] + (lo[b][i] + bx[i]));
+          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, bx[i]), sg);
           phi += r.y * w2[i];
           pb[b][i] = gphi * r.y;
           gv[b][i] = gphi * w2[i] * r.d;
@@ -487,6 +497,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       }
       gq = split_chunk(gv[0], gv[1]);
       put_slot(sz, l, gq);
+      phi *= sg;
       phi += shfl_xor(phi, 16);
       phi += shfl_xor(phi, 32);
       sw2 += edge_sums8(pb[0], pb[1], c);
@@ -506,7 +517,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       for (int b = 0; b < 2; ++b) {
         f32x4 gm = zero4();
         if (valid) gm = load4_f32(gmsg + (int64_t)ri * a.sgm + 16 * b + 4 * g);
-        v[b] = (gm + (hi[b] + lo[b])) * s2[b];
+        v[b] = add_signed(gm, hi[b] + lo[b], sg) * s2[b];
       }
       sb2 += edge_sums8(v[0], v[1], c);
       ga2 = split_chunk(v[0], v[1]);
@@ -538,7 +549,8 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
     }
     if constexpr (U) {
       wave_sync();
-      const Quad3 B0 = flip3(get_slot(sz, 0, c, g), flip), B1 = flip3(get_slot(sz, 1, c, g), flip);
+      const uint32_t fu = flip ^ 0x80000000u;   // g_a1 has no sign: the odd edges' inputs lose theirs
+      const Quad3 B0 = flip3(get_slot(sz, 0, c, g), fu), B1 = flip3(get_slot(sz, 1, c, g), fu);
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb) mma3e(gwu[hb][0], gwu[hb][1], get_slot(sx + (hb >> 1) * kSlot, hb & 1, c, g), B0, B1);
       wave_sync();

@@ -85,6 +85,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
 
   const uint32_t flip = g.partial ? (blockIdx.z & 1) << 31 : 0u;   // every other K range (flip_sign)
   const float sgn = flip ? -1.0f : 1.0f;
+  const uint32_t odd = g.partial ? 0u : 1u << 31;   // without splits: every other row of A
 
   struct Regs { f32x4 a[TA::nv], b[TB::nv]; };
   auto load = [&](int64_t k0, Regs& r) {
@@ -151,7 +152,16 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
       bf16* sa = s_a[u & 1];
       bf16* sb = s_b[u & 1];
 #pragma unroll
-      for (int i = 0; i < TA::nv; ++i) TA::put(sa, i, r[u].a[i]);
+      for (int i = 0; i < TA::nv; ++i) {
+        f32x4 v = r[u].a[i];
+        if constexpr (A_KC) {
+          v = flip_sign(v, TA::row(i) & 1 ? odd : 0u);
+        } else {   // rows 4 q .. 4 q + 3
+          v[1] = bitsf(fbits(v[1]) ^ odd);
+          v[3] = bitsf(fbits(v[3]) ^ odd);
+        }
+        TA::put(sa, i, v);
+      }
 #pragma unroll
       for (int i = 0; i < TB::nv; ++i) {
         TB::put(sb, i, flip_sign(r[u].b[i], flip));
@@ -180,6 +190,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
       const int64_t n = n0 + 32 * wn + 16 * j + 4 * gq;
       if (n >= g.N) continue;
       f32x4 v = hi[i][j] + lo[i][j];
+      if (!g.partial && (c & 1)) v = -v;
       if (g.partial) {
         *reinterpret_cast<f32x4*>(g.partial + ((int64_t)blockIdx.z * g.M + m) * g.N + n) = sgn * v;
         continue;

@@ -81,9 +81,12 @@ __device__ __forceinline__ void mma3x2(f32x4* hi, f32x4* lo, const Chunk3& a, co
   mma(lo[1], d.p0, b.p1);
 }
 
-// The matrix instruction drops the low bits of its sums towards one side, so the errors of many partial sums of one
-// result add up instead of averaging out.  Reductions over edges or nodes therefore contract with -B in every other
-// part and subtract: flip is the sign bit to change in B, sgn the factor of the part's result.
+// The matrix instruction drops the low bits of its sums towards one side, so the errors of many results of one kind add up
+// instead of averaging out where those are summed.  Reductions over edges or nodes therefore contract with -B in every
+// other part and subtract: flip is the sign bit to change in B, sgn the factor of the part's result.  The chains of the
+// edge kernels carry every other edge, and the node products every other row, with its sign changed (sg = -1): an edge's
+// operand is sg y, its products come out as sg times the sum, and sg goes back in by the multiplication or the signed
+// SiLU that follows, at no extra instruction.
 __device__ __forceinline__ f32x4 flip_sign(const f32x4& v, uint32_t flip) {
   f32x4 r;
 #pragma unroll
@@ -95,18 +98,26 @@ __device__ __forceinline__ f32x4 flip_sign(const f32x4& v, uint32_t flip) {
 // product's by fma, and log2 e's own), so the exponential keeps the accuracy of v_exp_f32 (1 ulp) for every x.
 // x is clamped in the exponent only, where the sigmoid is 0 or 1 to fp32 precision: an infinite x then gives
 // no inf - inf in d (SiLU(inf) = inf, SiLU(-inf) = -inf * 0 = NaN as with expf).
-__device__ __forceinline__ float sigmoid_f32(float x) {
+// signed forms, sg = 1 or -1: sg sigmoid(x), sg SiLU(x), sg SiLU'(x)
+__device__ __forceinline__ float sigmoid_f32(float x, float sg = 1.0f) {
   const float u = __builtin_amdgcn_fmed3f(x, -120.0f, 120.0f);
   const float t = u * -1.44269502e+0f;                                   // fl(log2 e)
   const float d = __builtin_fmaf(u, -1.92596303e-8f, __builtin_fmaf(u, -1.44269502e+0f, -t));
   const float e = __builtin_amdgcn_exp2f(t);
-  return __builtin_amdgcn_rcpf(1.0f + e * __builtin_fmaf(d, 0.693147182f, 1.0f));   // e may be inf: a product, no fma
+  return __builtin_amdgcn_rcpf(__builtin_fmaf(e * __builtin_fmaf(d, 0.693147182f, 1.0f), sg, sg));   // e may be inf: a product first
 }
-__device__ __forceinline__ float silu_f32(float x) { return x * sigmoid_f32(x); }
-__device__ __forceinline__ YD silu_yd_f32(float x) {
-  const float s = sigmoid_f32(x);
+__device__ __forceinline__ float silu_f32(float x, float sg = 1.0f) { return x * sigmoid_f32(x, sg); }
+__device__ __forceinline__ YD silu_yd_f32(float x, float sg = 1.0f) {
+  const float s = sigmoid_f32(x, sg);
   const float y = x * s;
-  return YD{y, __builtin_fmaf(y, 1.0f - s, s)};
+  return YD{y, __builtin_fmaf(y, __builtin_fmaf(s, -sg, 1.0f), s)};
+}
+// v + sg x
+__device__ __forceinline__ f32x4 add_signed(const f32x4& v, const f32x4& x, float sg) {
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_fmaf(x[i], sg, v[i]);
+  return r;
 }
 
 }  // namespace split

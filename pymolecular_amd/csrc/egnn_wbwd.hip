@@ -29,23 +29,6 @@ using namespace tile;
 constexpr int kWaves = 8, H = 256, O = 256, M = 256, KH = H / 32, kRB = 4, kST = H / (16 * kRB);   // kST chunks a stage
 constexpr int kChunkElems = kRB * KH * kFragElems;
 
-// v[j] and v[j + N] of two lanes -> the sum of one of them in each: N values left
-template <int DPP, int N> __device__ __forceinline__ void halve(float* v, bool up) {
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const float keep = up ? v[j + N] : v[j], send = up ? v[j] : v[j + N];
-    v[j] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), DPP, 0xf, 0xf, false));
-  }
-}
-// 16 values a lane, summed over the 16 edges (lanes c): lane c keeps value c
-__device__ __forceinline__ float edge_sum16(float* v, int c) {
-  halve<0x128, 8>(v, c & 8);   // row_ror:8
-  halve<0x141, 4>(v, c & 4);   // row_half_mirror
-  halve<0x4E, 2>(v, c & 2);    // quad_perm [2, 3, 0, 1]
-  halve<0xB1, 1>(v, c & 1);    // quad_perm [1, 0, 3, 2]
-  return v[0];
-}
-
 template <bool EQ, int NU>   // NU: 32-slot slices of the edge input (1 or 2)
 __global__ __launch_bounds__(64 * kWaves, 2) void wide_bwd_ep_kernel(BwdArgs a) {
   constexpr int NCH = (EQ ? 4 : 2) * kST;
