@@ -161,3 +161,33 @@ def test_small_width_many_tiles_per_wave():
     degs = np.full(3000, 29)
     rowptr, col = random_csr(len(degs), degs, seed=6)
     check_case(Case(rowptr, col, 32, 16, 64, 32, 32, seed=43, bias=False), "fp32")
+
+
+def test_stack_errors_do_not_add_up():
+    """Gradients of the coordinate MLPs of the first two of four layers (512 molecules, 12 seeds) against float64: sums of
+    190,000 terms of either sign, in which errors that point the same way for every edge add up.  Bound: their geometric
+    mean with the same layer on the fp32 matrix instruction, 6.0e-7 for these inputs (plain float32 torch: 1.9e-6; the
+    split products without the alternating signs: 8.8e-7)."""
+    from oracle import torch_ref
+    from pymolecular_amd import graphs
+    from pymolecular_amd.models.EGNN import EGNN
+    g = graphs.molecule_batch(512, seed=1001, feat_seed=3)
+    edges = [torch.from_numpy(g.rows().astype(np.int64)).cuda(), torch.from_numpy(g.col.astype(np.int64)).cuda()]
+    h = torch.from_numpy(g.node_feat).float().cuda()
+    logs = []
+    for seed in range(12):
+        torch.manual_seed(seed)
+        exact = torch_ref.EGNNRef(5, 128, 128, 0, n_layers=4).cuda()
+        ours = EGNN(5, 128, 128, 0, n_layers=4).cuda()
+        ours.load_state_dict({k.replace("layers.", "gcl_"): v for k, v in exact.state_dict().items()})
+        x, gx, gh = (1.5 * torch.randn(g.N, 3)).cuda(), torch.randn(g.N, 3).cuda(), torch.randn(g.N, 128).cuda()
+
+        def grads(m, layers, dt):
+            out = m(h.to(dt), x.to(dt), edges, None)
+            return torch.autograd.grad(out, [p for q in layers for p in q.coord_mlp.parameters()], [gh.to(dt), gx.to(dt)])
+        exact = exact.double()
+        got, want = grads(ours, [ours.gcl_0, ours.gcl_1], torch.float32), grads(exact, exact.layers[:2], torch.float64)
+        logs += [float(((a.double() - b).norm() / b.norm()).log()) for a, b in zip(got, want)]
+    err = float(np.exp(np.mean(logs)))
+    print("geometric mean of the errors:", err, flush=True)
+    assert err <= 6.1e-7
