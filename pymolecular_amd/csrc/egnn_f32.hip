@@ -146,7 +146,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
             const Chunk3 A = lds_chunk3((const bf16*)a.fr.s_u + ((int64_t)(rb >> 1) * 6 * a.NUC + ((rb & 1) * a.NUC + uc) * 3) * kFragElems, l);
             f32x4 lo = zero4(), hi = zero4();
             mma3(hi, lo, A, u3);
-            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], hi + lo, sg);
+            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], joined(hi, lo), sg);
           }
         }
       } else if constexpr (EQ) {
@@ -200,9 +200,9 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
         f32x4 x[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-          const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
+          const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g), p2 = joined(hi[b], lo[b]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) x[b][i] = silu_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
+          for (int i = 0; i < 4; ++i) x[b][i] = silu_f32(__builtin_fmaf(p2[i], sg, b2[i]), sg);
           *reinterpret_cast<f32x4*>(mrow + c * SP + 32 * (kp & 1) + 16 * b + 4 * g) = x[b];
         }
         stream_store((CH * kp + 1) & 1);
@@ -219,8 +219,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
             __builtin_amdgcn_sched_barrier(0);
             f32x4 lo3[2] = {zero4(), zero4()};
             mma3x2(q + rb, lo3, A.a, A.b, mc);
-            q[rb] += lo3[0];
-            q[rb + 1] += lo3[1];
+            q[rb] = joined(q[rb], lo3[0]);
+            q[rb + 1] = joined(q[rb + 1], lo3[1]);
             __builtin_amdgcn_sched_barrier(0);
             A = An;
           }
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       f32x4 lo = zero4();
       mma3(acc[rb], lo, A, B);
-      acc[rb] += lo;
+      acc[rb] = joined(acc[rb], lo);
       __builtin_amdgcn_sched_barrier(0);
       A = An;
       if (rb == 3) {
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
             const Chunk3 A = lds_chunk3((const bf16*)a.fr.s_u + ((int64_t)(rb >> 1) * 6 * a.NUC + ((rb & 1) * a.NUC + uc) * 3) * kFragElems, l);
             f32x4 lo = zero4(), hi = zero4();
             mma3(hi, lo, A, u3);
-            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], hi + lo, sg);
+            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], joined(hi, lo), sg);
           }
         }
       } else if constexpr (EQ) {
@@ -507,10 +507,10 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
       f32x4 x[2];
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
+        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g), p2 = joined(hi[b], lo[b]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
+          const YD r = silu_yd_f32(__builtin_fmaf(p2[i], sg, b2[i]), sg);
           x[b][i] = r.y;
           s2[kp][b][i] = r.d;
         }
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
         f32x4 hi[2] = {zero4(), zero4()}, lo[2] = {zero4(), zero4()};
         rows_chunk(2 * KP + 2 * kp, gq, hi, lo);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) x[b] = add_signed(x[b], hi[b] + lo[b], sg);
+        for (int b = 0; b < 2; ++b) x[b] = add_signed(x[b], joined(hi[b], lo[b]), sg);
       }
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
@@ -715,8 +715,9 @@ __global__ __launch_bounds__(kAtbThreads, 2) void atb_f32_kernel(AtbF32Args a) {
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
+        if (r == 0) hi[i][j] = joined(hi[i][j], lo[i][j]);
         float* o = P + (64 * wm + 16 * i + 4 * g + r) * 128 + 32 * wn + 16 * j + c;
-        const float v = sgn * (hi[i][j][r] + lo[i][j][r]);
+        const float v = sgn * hi[i][j][r];
         *o = a.add ? *o + v : v;
       }
   float* s = (float*)s_ab;   // [16][128] sums of the thread rows

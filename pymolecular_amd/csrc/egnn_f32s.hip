@@ -133,7 +133,7 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
 #pragma unroll
           for (int nb = 0; nb < 2; ++nb) mma3(hi[nb], lo[nb], A, u3[nb]);
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb) y[rb >> 1][nb][rb & 1] = add_signed(y[rb >> 1][nb][rb & 1], hi[nb] + lo[nb], sg);
+          for (int nb = 0; nb < 2; ++nb) y[rb >> 1][nb][rb & 1] = add_signed(y[rb >> 1][nb][rb & 1], joined(hi[nb], lo[nb]), sg);
         }
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
@@ -159,8 +159,9 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
       const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 16 * b + 4 * g);
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
+        const f32x4 p = joined(hi[nb], lo[nb]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[nb][b][i] = silu_f32(__builtin_fmaf(hi[nb][i] + lo[nb][i], sg, b2[i]), sg);
+        for (int i = 0; i < 4; ++i) x[nb][b][i] = silu_f32(__builtin_fmaf(p[i], sg, b2[i]), sg);
         *reinterpret_cast<f32x4*>(msg + (16 * nb + c) * SP + 16 * b + 4 * g) = x[nb][b];
       }
     }
@@ -179,9 +180,11 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
         const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 16 * b + 4 * g);
         const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g);
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
+        for (int nb = 0; nb < 2; ++nb) {
+          const f32x4 p = joined(hi[nb], lo[nb]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) phi[nb] += silu_f32(__builtin_fmaf(hi[nb][i] + lo[nb][i], sg, bx[i])) * w2[i];
+          for (int i = 0; i < 4; ++i) phi[nb] += silu_f32(__builtin_fmaf(p[i], sg, bx[i])) * w2[i];
+        }
       }
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
@@ -295,7 +298,7 @@ __device__ __forceinline__ Quad3 get_slot(const bf16* s, int blk, int c, int g) 
   auto one = [&](const bf16* q) { return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)q); };
   return Quad3{one(p), one(p + kFragElems), one(p + 2 * kFragElems)};
 }
-// acc += A^T B over the 16 edges: the corrections, then the large term
+// acc += A^T B over the 16 edges: the corrections, then the large term (one accumulator, so an infinite operand gives NaN)
 __device__ __forceinline__ void mma16(f32x4& acc, const bf16x4& a, const bf16x4& b) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), acc, 0, 0, 0);
@@ -436,8 +439,8 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         for (int rb = 0; rb < 4; rb += 2) {
           f32x4 hi[2] = {zero4(), zero4()}, lo[2] = {zero4(), zero4()};
           mma3x2(hi, lo, frag3(s_u + rb * 3 * kFragElems, l), frag3(s_u + (rb + 1) * 3 * kFragElems, l), u3);
-          y[rb] = add_signed(y[rb], hi[0] + lo[0], sg);
-          y[rb + 1] = add_signed(y[rb + 1], hi[1] + lo[1], sg);
+          y[rb] = add_signed(y[rb], joined(hi[0], lo[0]), sg);
+          y[rb + 1] = add_signed(y[rb + 1], joined(hi[1], lo[1]), sg);
         }
         opaque(u.lo);   // split again for d[W_e | w_d]
         opaque(u.hi);
@@ -465,10 +468,10 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         mma3x2(hi, lo, w_cols3<H>(s_hl, 0, kc, c, g), w_cols3<H>(s_hl, 1, kc, c, g), m1[kc]);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 16 * b + 4 * g);
+        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 16 * b + 4 * g), p = joined(hi[b], lo[b]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
+          const YD r = silu_yd_f32(__builtin_fmaf(p[i], sg, b2[i]), sg);
           x[b][i] = r.y;
           s2[b][i] = r.d;
         }
@@ -486,10 +489,10 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 16 * b + 4 * g);
-        const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g);
+        const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g), p = joined(hi[b], lo[b]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, bx[i]), sg);
+          const YD r = silu_yd_f32(__builtin_fmaf(p[i], sg, bx[i]), sg);
           phi += r.y * w2[i];
           pb[b][i] = gphi * r.y;
           gv[b][i] = gphi * w2[i] * r.d;
@@ -517,7 +520,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       for (int b = 0; b < 2; ++b) {
         f32x4 gm = zero4();
         if (valid) gm = load4_f32(gmsg + (int64_t)ri * a.sgm + 16 * b + 4 * g);
-        v[b] = add_signed(gm, hi[b] + lo[b], sg) * s2[b];
+        v[b] = add_signed(gm, joined(hi[b], lo[b]), sg) * s2[b];
       }
       sb2 += edge_sums8(v[0], v[1], c);
       ga2 = split_chunk(v[0], v[1]);
@@ -537,7 +540,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
       mma3x2(hi, lo, w_rows3<H>(s_hl, 2 * kc, c, g), w_rows3<H>(s_hl, 2 * kc + 1, c, g), ga2);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        v[b] = (hi[b] + lo[b]) * s1[2 * kc + b];
+        v[b] = joined(hi[b], lo[b]) * s1[2 * kc + b];
         if (valid) *reinterpret_cast<f32x4*>((float*)a.Gh + (ee - a.gbase) * H + 32 * kc + 16 * b + 4 * g) = v[b];
         if constexpr (EQ) {
           const f32x4 wd = *reinterpret_cast<const f32x4*>(s_vec + O + 2 * M + 32 * kc + 16 * b + 4 * g);

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32s_kernel(Gemm2Args g) {
     for (int j = 0; j < NJ; ++j) {
       const int64_t n = n0 + 32 * wn + 16 * j + 4 * gq;
       if (n >= g.N) continue;
-      f32x4 v = hi[i][j] + lo[i][j];
+      f32x4 v = joined(hi[i][j], lo[i][j]);
       if (!g.partial && (c & 1)) v = -v;
       if (g.partial) {
         *reinterpret_cast<f32x4*>(g.partial + ((int64_t)blockIdx.z * g.M + m) * g.N + n) = sgn * v;

@@ -9,9 +9,10 @@
 // are exact in fp32.  The large term has an accumulator of its own (K / 32 roundings instead of the K / 4 or
 // more of the fp32 instruction); the five correction terms, 2^-8 of it or less, go to a second one.
 //
-// An infinite operand has no such parts (inf - inf), so the products it enters are NaN where the fp32
-// instruction may give an infinity; a finite one never becomes infinite (x0 is truncated), and a column of
-// the result that no such operand enters is not touched.
+// An infinite operand has no such parts: its second is inf - inf = NaN, which enters the correction terms only.  The two
+// accumulators are therefore added by joined(), which takes the large term alone where the corrections are NaN, so an
+// infinity comes out where the fp32 instruction gives one.  (Not in the weight gradients of egnn_f32s.hip, which keep both
+// in one accumulator: NaN there.)  A finite operand never becomes infinite, as x0 is truncated.
 #pragma once
 #include "egnn_device.h"
 
@@ -79,6 +80,16 @@ __device__ __forceinline__ void mma3x2(f32x4* hi, f32x4* lo, const Chunk3& a, co
   mma(lo[1], d.p1, b.p0);
   mma(lo[0], a.p0, b.p1);
   mma(lo[1], d.p0, b.p1);
+}
+
+// hi + lo, and hi alone where lo is NaN.  lo is NaN exactly where an infinite (or NaN) operand entered the sum, as such an
+// operand has no second and third part; hi is then what the fp32 product gives.
+__device__ __forceinline__ f32x4 joined(const f32x4& hi, const f32x4& lo) {
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    r[i] = hi[i] + __builtin_amdgcn_fmed3f(lo[i], -3.40282347e+38f, lo[i]);   // NaN -> the finite bound: one instruction
+  return r;
 }
 
 // The matrix instruction drops the low bits of its sums towards one side, so the errors of many results of one kind add up

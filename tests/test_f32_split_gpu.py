@@ -191,3 +191,43 @@ def test_stack_errors_do_not_add_up():
     err = float(np.exp(np.mean(logs)))
     print("geometric mean of the errors:", err, flush=True)
     assert err <= 6.1e-7
+
+
+@pytest.mark.parametrize("eq", [True, False])
+@pytest.mark.parametrize("dims", [(128, 128, 128), (64, 32, 32)])
+def test_infinite_operands(dims, eq):
+    """Infinities come out where the float64 oracle has them, in the forward (an infinite bias of the first layer: each
+    message feature is infinite or, as SiLU(-inf), NaN) and in the gradients (an infinite message gradient)."""
+    H, O, M = dims
+    degs = [0] * 20 + _degrees("halves")
+    rowptr, col = random_csr(len(degs), degs, seed=8)
+    case = Case(rowptr, col, 32, 8, H, O, M, seed=45, eq=eq)
+    case.p["b1"][H - 3] = np.inf
+    got = run_fused(case, "fp32", backward=False)["out_msg"]
+    live = np.diff(rowptr) > 0
+    up = case.p["w2_msg"][H - 3] > 0
+    assert np.isposinf(got[live][:, up]).all() and np.isnan(got[live][:, ~up]).all() and (got[~live] == 0).all()
+
+    case = Case(rowptr, col, 32, 8, H, O, M, seed=46, eq=eq)
+    row, o = int(np.flatnonzero(np.diff(rowptr) == 1)[0]), 5     # a row of one edge: its gradient reaches one source
+    case.gm[row, o] = np.inf
+    want = case.backward_ref(False)
+    res = run_fused(case, "fp32")["grads"]
+    assert not np.isfinite(want["b1"]).any() and np.array_equal(np.sign(res["b1"]), np.sign(want["b1"]))
+    assert np.isinf(res["b1"]).all()
+    w2, ref = res["w2_msg"].reshape(H, O), want["w2_msg"].reshape(H, O)
+    assert np.isfinite(np.delete(w2, o, 1)).all() and not np.isfinite(w2[:, o]).any()
+    if H == 128:   # at H = 64 the large term and the corrections share an accumulator: NaN
+        assert np.array_equal(w2[:, o], ref[:, o])
+
+
+@pytest.mark.parametrize("N", [5, 4100])
+def test_infinite_rows_of_node_products(N):
+    from pymolecular_amd.node_update import dense
+    torch.manual_seed(N)
+    lin = torch.nn.Linear(128, 64).cuda()
+    x = torch.randn(N, 128).cuda()
+    x[3, 7] = float("inf")
+    x.requires_grad_()
+    y = dense(x, lin)
+    assert torch.equal(y[3], torch.sign(lin.weight[:, 7]) * float("inf")) and torch.isfinite(y).sum() == (N - 1) * 64
