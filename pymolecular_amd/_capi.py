@@ -64,19 +64,19 @@ _lib = None
 ABI_VERSION = 9   # include/egnn.h egnn_abi_version()
 
 
-def _check_stamp() -> None:
+def _check_stamp(path=None, stamp=None, digest=None, what="other sources") -> None:
     """Refuse a library that was not built from the sources in this tree.
 
-    The build writes the SHA-256 of its sources next to the library; a missing
-    or different stamp means the library is stale (or foreign)."""
+    The build writes the SHA-256 of what it was built from next to the library;
+    a missing or different stamp means the library is stale (or foreign).
+    Default: the HIP library."""
     from . import _build
-    stamp = _build.STAMP
+    path, stamp, digest = path or LIB_PATH, stamp or _build.STAMP, digest or _build.source_hash
     if not stamp.exists():
         raise RuntimeError(f"{stamp} is missing: rebuild the library with `python -m pymolecular_amd._build`")
-    built = stamp.read_text().strip()
-    now = _build.source_hash()
+    built, now = stamp.read_text().strip(), digest()
     if built != now:
-        raise RuntimeError(f"{LIB_PATH} was built from other sources (sha256 {built[:16]}, tree {now[:16]}): "
+        raise RuntimeError(f"{path} was built from {what} (sha256 {built[:16]}, now {now[:16]}): "
                            "rebuild it with `python -m pymolecular_amd._build`")
 
 
@@ -161,11 +161,18 @@ _ext = None
 
 
 def ext():
-    """The native autograd node of the layer (csrc/egnn_torch.cpp), loaded once; raises if it has not been built."""
+    """The native autograd node of the layer (csrc/egnn_torch.cpp), loaded once; raises if it has not been built, or
+    was built from other sources or against another torch, C++ ABI or Python."""
     global _ext
     if _ext is None:
         import torch  # noqa: F401  (its libraries, which the module links to)
+
+        from . import _build
         lib()         # built from these sources
+        if not _build.EXT.exists():
+            raise RuntimeError(f"{_build.EXT} is missing: build it with `python -m pymolecular_amd._build` "
+                               "(or __graft_entry__.build())")
+        _check_stamp(_build.EXT, _build.EXT_STAMP, _build.ext_hash, "other sources or against another torch or Python")
         from . import _egnn_torch
         _ext = _egnn_torch
     return _ext
