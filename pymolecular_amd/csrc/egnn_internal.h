@@ -21,7 +21,6 @@ struct SchedView {
   int32_t* n_fix;     // [1]
   int32_t* csc_ptr;   // [N+1] source-sorted offsets
   int32_t* csc_eid;   // [E]   CSR edge positions sorted by col (stable)
-  int32_t* err;       // [1]   CSR validation flag
   int32_t* tile_tab;  // [ceil(E/32)][64] ranks of each 32-edge tile (kTab* offsets)
 };
 // Ranks of a 32-edge tile (the maximal runs of edges of one row inside it), one 64-int row per tile:

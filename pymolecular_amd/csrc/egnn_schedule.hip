@@ -28,7 +28,6 @@ size_t sched_layout(int64_t N, int64_t E, void* base, SchedView* v) {
   v->n_fix = (int32_t*)take(sizeof(int32_t));
   v->csc_ptr = (int32_t*)take(sizeof(int32_t) * (size_t)(N + 1));
   v->csc_eid = (int32_t*)take(sizeof(int32_t) * (size_t)std::max<int64_t>(E, 1));
-  v->err = (int32_t*)take(sizeof(int32_t));
   v->tile_tab = (int32_t*)take(sizeof(int32_t) * kTabInts * (size_t)std::max<int64_t>(cdiv(E, kTileEdges), 1));
   return off;
 }

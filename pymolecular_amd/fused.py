@@ -60,10 +60,9 @@ def schedule_arrays(sched: Schedule) -> dict:
     off = 0
     out = {}
     for name, n in (("erow", max(E, 1)), ("fix_rows", N), ("n_fix", 1), ("csc_ptr", N + 1), ("csc_eid", max(E, 1)),
-                    ("err", 1), ("tile_tab", ntiles * 64)):
+                    ("tile_tab", ntiles * 64)):
         out[name] = sched.buf[off:off + 4 * n].view(torch.int32)
         off = (off + 4 * n + 255) // 256 * 256
-    out.pop("err")
     out["tile_tab"] = out["tile_tab"].view(ntiles, 64)[:(E + 31) // 32]
     nf = int(out.pop("n_fix")[0])
     out["fix_rows"] = out["fix_rows"][:nf]

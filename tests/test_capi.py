@@ -137,6 +137,15 @@ def test_identity_probe_flag_only_for_bf16_mpnn_h128():
     assert L.egnn_fwd_workspace_bytes(_capi.EgnnDims(**dict(big, flags=0))) > 0
 
 
+def test_schedule_holds_only_its_arrays():
+    # the six arrays of fused.schedule_arrays, each 256-byte aligned
+    L = _capi.lib()
+    for N, E in ((1, 0), (1, 1), (100, 3200), (70_000, 1_000_001)):
+        tiles = max((E + 31) // 32, 1)
+        sizes = (max(E, 1), N, 1, N + 1, max(E, 1), tiles * 64)
+        assert L.egnn_schedule_bytes(N, E) == sum((4 * n + 255) // 256 * 256 for n in sizes)
+
+
 def test_fp32_backward_scratch_is_bounded():
     # the fp32 backward keeps its per-edge rows (factors, dL/dpre1, dL/ddelta, r^2) one edge chunk at a
     # time: its workspace grows with the nodes, not with the edges, past the chunk budget
