@@ -155,8 +155,11 @@ def test_fp32_backward_scratch_is_bounded():
     big = L.egnn_bwd_workspace_bytes(_capi.EgnnDims(N=250_000, E=32_000_000, **kw))
     assert big - small < 32 << 20, (small >> 20, big >> 20)          # 4x the edges, about the same scratch
     assert small < (256 << 20) + 2 * 250_000 * 2 * 64 * 4 + (32 << 20), small >> 20   # chunk + node rows
-    # graphs of 8,192 edges or more take at least two chunks: the scratch is about half the per-edge state
-    one = L.egnn_bwd_workspace_bytes(_capi.EgnnDims(N=1000, E=8000, **kw))
-    two = L.egnn_bwd_workspace_bytes(_capi.EgnnDims(N=1000, E=32_000, **kw))
-    per_edge = (64 + 2 * 32 + 2 * 32) * 4 + 64 * 4 + 16 + 4
-    assert two < 0.6 * 32_000 * per_edge + one, (one, two)
+    # at these widths the kernels keep no factors: 272 bytes per edge (dL/dpre1, dL/ddelta), one chunk up to the budget
+    # of 256 MiB = 986,895 edges, two of half the edges past it
+    ws = lambda E: L.egnn_bwd_workspace_bytes(_capi.EgnnDims(N=1000, E=E, **kw))  # noqa: E731
+    assert ws(900_000) - ws(200_000) == 700_000 * 272
+    assert ws(986_880) > 986_880 * 272 and ws(986_912) < 0.6 * ws(986_880)
+    # H = 128 on split operands: four factors of 128 as well, 2,576 bytes per edge, two chunks from 65,536 edges on
+    kw.update(F=128, FE=0, H=128, O=128, M=128)
+    assert ws(65_504) > 65_504 * 2576 and ws(65_536) < 0.6 * ws(65_504)

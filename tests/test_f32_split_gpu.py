@@ -122,7 +122,7 @@ def _gemm_case(N, K1, K2, Hn, Fo, res, seed):
     (33, 8, 8, 24, 8, True),             # K of 16 and 24: a slice's tail, columns past N
     (65, 128, 128, 128, 128, False),
     (257, 40, 24, 72, 48, False),        # no multiple of a tile anywhere
-    (8200, 128, 128, 128, 128, True),    # 64-row tiles
+    (8200, 128, 128, 128, 128, True),    # 256 tiles and a remainder; 64-row tiles in the weight gradients
     (4099, 136, 120, 256, 136, True),    # concatenation inside a 32-deep slice
 ])
 def test_f32_node_products(N, K1, K2, Hn, Fo, res):

@@ -229,9 +229,9 @@ def test_egnn_forward_many_tiles_per_wave():
 @pytest.mark.parametrize("dims,eq,mean", [((32, 16, 64, 32, 32), True, False), ((128, 16, 128, 128, 128), True, True),
                                            ((128, 24, 128, 128, 128), False, False)])
 def test_fp32_edge_chunks(dims, eq, mean):
-    """The fp32 backward in edge chunks (more than 8,192 edges: at least two; Gh, Gx, r^2 and the factors
-    held one chunk at a time, the node sums and weight gradients added in chunk order): rows that straddle
-    the chunk boundaries, empty rows, a degree-1,500 row, edge ids that permute the feature rows."""
+    """The fp32 backward at 103,680 edges: at H = 128 two edge chunks (Gh, Gx and the factors held one chunk at a
+    time, the node sums and weight gradients added in chunk order), at H = 64 one (two: test_fp32_small_width_chunks).
+    Rows that straddle the chunk boundary, empty rows, a degree-1,500 row, edge ids that permute the feature rows."""
     from pymolecular_amd import _capi
     F, FE, H, O, M = dims
     degs = np.array([0, 1500, 3, 61, 0, 7, 33, 2, 90, 1, 31] * 60)
@@ -242,6 +242,39 @@ def test_fp32_edge_chunks(dims, eq, mean):
     print(f"[fp32-chunks] N={len(degs)} E={E} dims={dims} eq={eq} mean={mean} "
           f"workspace {_capi.lib().egnn_bwd_workspace_bytes(d) / 2 ** 20:.1f} MB", flush=True)
     check_case(Case(rowptr, col, F, FE, H, O, M, seed=97, eq=eq, mean_agg=mean, edge_ids=perm), "fp32")
+
+
+@pytest.mark.parametrize("eq", [True, False])
+def test_fp32_small_width_chunks(eq):
+    """H = 64 past the 986,895 edges that fit one chunk: the second chunk adds to the first one's partial rows and node
+    sums.  Against the sum, in float64, of the backwards of two parts of the rows, each of one chunk; a row across the
+    chunk boundary, a last chunk that ends inside a tile, edge ids that permute the feature rows.  Each of the three runs
+    is within 1e-5 of the exact result (the bound of every fp32 test here)."""
+    from pymolecular_amd import _capi
+    F, FE, H, O, M = 32, 16, 64, 32, 32
+    degs = np.array([0, 1500, 3, 61, 0, 7, 33, 2, 90, 1, 31] * 579 + [5])
+    rowptr, col = random_csr(len(degs), degs, seed=98)
+    E = len(col)
+    dims = lambda e: _capi.EgnnDims(N=len(degs), E=e, F=F, FE=FE, H=H, O=O, M=M, equivariant=int(eq), mean_agg=1, dtype=0)  # noqa: E731
+    ws = _capi.lib().egnn_bwd_workspace_bytes
+    assert E % 32 and E > 986_895 and ws(dims(E)) < 0.6 * ws(dims(986_880))     # two chunks
+    half = -(-(-(-E // 2)) // 32) * 32
+    assert half not in rowptr                                                   # a row across the boundary
+    r = np.random.Generator(np.random.PCG64(99))
+    case = Case(rowptr, col, F, FE, H, O, M, seed=100, eq=eq, mean_agg=True, edge_ids=r.permutation(E))
+    got = run_fused(case, "fp32")["grads"]
+    cut = int(np.searchsorted(rowptr, 300_000))
+    parts = []
+    for lo, hi in ((0, cut), (cut, len(degs))):
+        part = Case(np.clip(rowptr, rowptr[lo], rowptr[hi]) - rowptr[lo], col[rowptr[lo]:rowptr[hi]], F, FE, H, O, M,
+                    seed=100, eq=eq, mean_agg=True, edge_ids=np.arange(rowptr[hi] - rowptr[lo]))
+        part.h, part.coord, part.p, part.gm, part.gx = case.h, case.coord, case.p, case.gm, case.gx
+        part.ef = case.ef[case.edge_ids[rowptr[lo]:rowptr[hi]]]
+        parts.append(run_fused(part, "fp32")["grads"])
+    for k, v in got.items():
+        if v is not None:
+            err = orc.normwise_rel_err(v, parts[0][k].astype(np.float64) + parts[1][k])
+            assert err <= 2e-5, (k, err)
 
 
 def test_mpnn_forward_wide_message_rows():
