@@ -572,8 +572,8 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
   __syncthreads();
   float* const sum = (float*)s_x;   // [dW_hl | db2 | dW1_mov | dbx1 | dw2_mov | dW_e | dw_d]
   constexpr int oB2 = H * O, oM = oB2 + O, oBx = oM + (EQ ? O * M : 0), oW2 = oBx + (EQ ? M : 0), oE = oW2 + (EQ ? M : 0);
-  const int FE = a.FE, LW = oE + H * FE + (EQ ? H : 0);   // at most 5,344 floats (F_E = 32)
-  static_assert((oE + H * 33) * sizeof(float) <= sizeof(s_x), "the partial row fits the exchange buffers");
+  const int FE = a.FE, LW = oE + H * FE + (EQ ? H : 0);   // at most 4,768 floats (EGNN, F_E = 24)
+  static_assert((oE + H * 33) * sizeof(float) <= sizeof(s_x), "the partial row fits the exchange buffers");   // 32 slots and w_d
   for (int q = 0; q < kW; ++q) {
     if (w == q) {
       auto add = [&](int i, float v) { sum[i] = q ? sum[i] + v : v; };

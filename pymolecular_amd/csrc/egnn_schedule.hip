@@ -36,9 +36,11 @@ size_t sched_layout(int64_t N, int64_t E, void* base, SchedView* v) {
 // list, kSortMax / 64 values per lane).
 constexpr int kScanRows = 2048, kSortMax = 512;
 // The counting path counts the edges per source by atomics, scatters one 4-byte id per edge and sorts each node's
-// list in registers: 334 k edges 36 us in four launches against 120 us in 24 with the library's sort.  Past these
-// many edges the atomics cost more than they save (0.88M edges of a power-law graph: a first pass 1.09 against
-// 1.03 ms; 11.6M edges: 0.7 ms longer for the count alone).
+// list in registers: 334 k edges 36 us in four launches against 120 us in 24 with the library's sort.  The scatter's
+// cost grows with the spread of the sources, so the two cross between 0.9M and 2M edges by kind of graph; the line lies
+// below all of them.  One schedule, counting / sort: chains with kNN edges 983k 120 / 213 us, 1.97M 173 / 174, 3.9M
+// 278 / 257; random sources 1.28M 251 / 165, 2.56M 422 / 179; power law 0.87M 193 / 253, 1.40M 273 / 210, and with the
+// hubs as sources (lists past kSortMax: counted in vain, then sorted) 0.87M 290 / 243.
 constexpr int64_t kCountMaxEdges = int64_t(3) << 18;
 
 struct SchedTmp {

@@ -4,8 +4,9 @@
 // is done as six bf16 products.  A value x is split into three bf16 parts that carry its 24 significand
 // bits exactly: x0 = the upper 16 bits of x (never overflows), x1 = bf16(x - x0), x2 = x - x0 - x1 (both
 // differences are exact, and the last one has at most 8 bits).  a b is then a0 b0 + (a0 b1 + a1 b0) +
-// (a0 b2 + a1 b1 + a2 b0); what is left out, a1 b2 + a2 b1 + a2 b2, is below 2^-23 |a b| at worst and
-// about 2^-27 |a b| rms, of either sign, against the 2^-25 rms of one fp32 rounding.  The bf16 products
+// (a0 b2 + a1 b1 + a2 b0); what is left out, a1 b2 + a2 b1 + a2 b2, is below 2^-22 |a b| at worst
+// (a = b = 1.0078) and 2^-25.5 |a b| rms over all significands, about one fp32 rounding of that product; the
+// fp32 instruction rounds the growing sum instead, K times.  The bf16 products
 // are exact in fp32.  The large term has an accumulator of its own (K / 32 roundings instead of the K / 4 or
 // more of the fp32 instruction); the five correction terms, 2^-8 of it or less, go to a second one.
 //
