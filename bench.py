@@ -123,9 +123,12 @@ def kernel_work(cls, path, N, E, F, H, O, M, FE, g, s):
         elif path == "wide":  # factors m1, m, g_q, g_a2 stored for the split-K products (dw2_mov, dw_d in the kernel)
             flops = 2 * (g + FE) * H + 4 * H * O + 4 * g * O * M
             per_edge += (H + O + g * M + O) * s
-        else:                 # fp32 on split operands: the same factors; dw2_mov, dw_d and dW_e in the kernel
-            flops = 4 * (g + FE) * H + 4 * H * O + 4 * g * O * M
+        elif path == "split":  # fp32, H = 128, on split operands: the same factors; dw2_mov and dw_d in the kernel
+            flops = (4 * g + 2 * FE) * H + 4 * H * O + 4 * g * O * M
             per_edge += (H + O + g * M + O) * s
+        else:         # one wave per tile (fp32, H = 256): factors m1, m, g_q, p, g_a2 and r^2 stored
+            flops = 2 * (g + FE) * H + 4 * H * O + 4 * g * O * M
+            per_edge += (H + O + 2 * g * M + O) * s + 4 * g
         if dst:
             return flops * E, E * (per_edge + H / 4) + N * H * s
         return flops * E, E * per_edge
@@ -142,9 +145,12 @@ def kernel_work(cls, path, N, E, F, H, O, M, FE, g, s):
         if path == "wide":     # [dW_hl; db2], [dW1_mov; dbx1] over the edge factors; dW_e over Gh
             flops = 2 * E * ((H + 1) * O + g * (O + 1) * M + H * FE)
             nbytes = E * ((H + O) * s + g * (O + M) * s + (H * s + FE * s + 4 if FE else 0))
-        elif path == "split":  # [dW_hl; db2], [dW1_mov; dbx1] over the edge factors
-            flops = 2 * E * ((H + 1) * O + g * (O + 1) * M)
-            nbytes = E * ((H + O) * s + g * (O + M) * s)
+        elif path == "split":  # the same products
+            flops = 2 * E * ((H + 1) * O + g * (O + 1) * M + H * FE)
+            nbytes = E * ((H + O) * s + g * (O + M) * s + (H * s + FE * s + 4 if FE else 0))
+        elif path == "one":    # and the dw2_mov and dw_d matrix-vector products over p, Gh and r^2
+            flops = 2 * E * ((H + 1) * O + g * ((O + 1) * M + M + H) + H * FE)
+            nbytes = E * ((H + O) * s + g * ((O + M) * s + M * s + 4 + H * s + 4) + (H * s + FE * s + 4 if FE else 0))
         return flops, nbytes
     return 0, 0
 
@@ -313,7 +319,8 @@ def run_workload(k, dtype, a, g=None):
 
     s = 2 if dt == torch.bfloat16 else 4
     g1 = 1 if eq else 0
-    path = "coop" if s == 2 and H == 128 and FE + 2 * g1 <= 32 else "wide" if s == 2 and H == 256 else "split"
+    path = "coop" if s == 2 and H == 128 and FE + 2 * g1 <= 32 else "wide" if s == 2 and H == 256 else \
+        "split" if s == 4 and H == 128 else "one"
     peak_mfma = PEAK["bf16_mfma_tflops"] if s == 2 else PEAK["fp32_mfma_tflops"]
 
     def executed_per_launch(cls, launches_per_step):
