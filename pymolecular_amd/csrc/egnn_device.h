@@ -110,6 +110,8 @@ __device__ __forceinline__ f32x4 load4_f32(const bf16* p) {
 constexpr uint32_t kOob = 0x80000000u;   // a buffer offset past every buffer
 constexpr int kBufFlags = 0x00020000;    // buffer resource word 3 (gfx9 family): raw, range-checked
 
+__device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
+
 // ---- activations ---------------------------------------------------------
 // SiLU(x) = x / (1 + e^-x), written from the definition; sigma is kept so the
 // backward gets SiLU'(x) = sigma * (1 + x (1 - sigma)) for a few more flops.
@@ -131,6 +133,12 @@ template <typename T> __device__ __forceinline__ YD silu_yd(float x) {
 
 // ---- wave helpers --------------------------------------------------------
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+// a wave's own LDS writes before its lanes' reads of each other's, and back
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 __device__ __forceinline__ float shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }
 __device__ __forceinline__ float shfl(float v, int src) { return __shfl(v, src, 64); }
 __device__ __forceinline__ int shfl_i(int v, int src) { return __shfl(v, src, 64); }

@@ -98,12 +98,6 @@ __global__ __launch_bounds__(64 * kEqWaves, 1) void egnn_fwd_ep_kernel(FwdArgs a
     for (int rb = 0; rb < NRB; ++rb) asm volatile("" ::"v"(d.pq[rb]));
     asm volatile("" ::"v"(d.u), "v"(x.ri), "v"(x.rj), "v"(x.eid));
   };
-  // a wave's LDS writes seen by its other lanes (the waves never read each other's rows)
-  auto wave_sync = [&]() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
 
   bf16* const msgw = s_msg[w];
   // One 16-edge half h of tile T: S1 on cur, then the gathers of the half after it (indices xn) into

@@ -27,7 +27,6 @@ using namespace split;
 
 constexpr int kF32Waves = 4;
 
-__device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 __device__ __forceinline__ Chunk3 lds_chunk3(const bf16* frag, int l) {
   const bf16* p = frag + l * 8;
   return Chunk3{load_chunk(p), load_chunk(p + kFragElems), load_chunk(p + 2 * kFragElems)};
@@ -45,11 +44,6 @@ struct RowAddr {
 // fragments of two row blocks
 struct Pair3 { Chunk3 a, b; };
 __device__ __forceinline__ Pair3 pair3(const bf16* a, const bf16* b, int l) { return Pair3{lds_chunk3(a, l), lds_chunk3(b, l)}; }
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 template <bool EQ, bool FEAT>
 __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {

@@ -18,7 +18,6 @@ namespace egnn {
 namespace {
 
 using namespace split;
-using tile::zero4;
 
 constexpr int kW = 4, H = 64, O = 32, M = 32, KH = H / 32;
 
@@ -36,11 +35,6 @@ __device__ __forceinline__ void split_frags(bf16* dst, const float* src, int nfr
 __device__ __forceinline__ Chunk3 frag3(const bf16* f, int l) {
   const bf16* p = f + l * 8;
   return Chunk3{load_chunk(p), load_chunk(p + kFragElems), load_chunk(p + 2 * kFragElems)};
-}
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 // r^2 and delta of an edge
 struct Geo { float dx, dy, dz, r2; };

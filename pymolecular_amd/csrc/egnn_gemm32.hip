@@ -21,7 +21,6 @@ using namespace split;
 
 constexpr int kBN = 64, kBK = 32, kRing = 4;
 
-__device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 __device__ __forceinline__ int chain_pos4(int f) {   // chain position of features f .. f + 3 of a 32-group (f % 4 = 0)
   return f < 16 ? 2 * f : 2 * (f - 16) + 4;
 }

@@ -20,7 +20,6 @@ __device__ __forceinline__ bf16x4 pack4(const f32x4& v) {
 __device__ __forceinline__ f32x4 unpack4(const bf16x4& v) {
   return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
 }
-__device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 
 // chain buffer over NB 16-edge blocks: chunk (kc, nb) = 64 lanes x 8 bf16 at index kc NB + nb;
 // 16-row block blk fills half (blk & 1) of chunk blk >> 1.  With SW the 16-byte lane slot s of a

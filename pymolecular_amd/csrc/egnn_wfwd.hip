@@ -66,11 +66,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void wide_fwd_ep_kernel(FwdArgs a) 
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<bf16x8*>(dst + i * 64 * kWaves * 8) = st[i];
   };
-  auto wave_sync = [&]() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
   // 32 rows (chunk ch) of a product with both edge blocks: acc[row block][edge block] += W . B
   auto rows = [&](int ch, const bf16x8 (*B)[2], f32x4 (*acc)[2]) {
     const bf16* W = s_w[ch & 1] + l * 8;
