@@ -92,8 +92,8 @@ __global__ __launch_bounds__(W * 64, 4) void coop_fwd_kernel(FwdArgs a) {
     }
   }
 #pragma unroll
-  for (int j = 0; j < BH; ++j)
-    wu[j] = load_chunk((const bf16*)a.fr.u + (int64_t)(w * BH + j) * kFragElems + l * 8);
+  for (int j = 0; j < BH; ++j)   // without edge inputs (MPNN, F_E = 0) there are no W_u fragments
+    wu[j] = EQ || FE > 0 ? load_chunk((const bf16*)a.fr.u + (int64_t)(w * BH + j) * kFragElems + l * 8) : zero_chunk<bf16>();
 #pragma unroll
   for (int j = 0; j < BO; ++j) {
 #pragma unroll
@@ -417,7 +417,8 @@ __global__ __launch_bounds__(W * 64) void coop_bwd_kernel(BwdArgs a) {
 #pragma unroll
   for (int j = 0; j < BH; ++j) {
     const int hb = w * BH + j;
-    wu[j] = load_chunk((const bf16*)a.fr.u + (int64_t)hb * kFragElems + l * 8);
+    // without edge inputs (MPNN, F_E = 0) there are no W_u fragments
+    wu[j] = EQ || NU > 0 ? load_chunk((const bf16*)a.fr.u + (int64_t)hb * kFragElems + l * 8) : zero_chunk<bf16>();
   }
 #pragma unroll
   for (int j = 0; j < BO; ++j) {

@@ -137,6 +137,14 @@ def test_mpnn_edge_parallel_cases(fe, skewed, eids):
     check_case(Case(rowptr, col, 128, fe, 128, 128, 128, seed=22 + fe, eq=False, edge_ids=perm), "bf16")
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("degs", [[2] * 9, [0, 300, 1, 2, 0, 129, 3, 31, 33]])
+def test_mpnn_h64_without_edge_features(degs, dtype):
+    """MPNN at H = 64 with F_E = 0: no edge input at all, so no W_u fragments exist."""
+    rowptr, col = random_csr(len(degs), degs, seed=62)
+    check_case(Case(rowptr, col, 32, 0, 64, 32, 32, seed=24, eq=False), dtype)
+
+
 @pytest.mark.parametrize("fe,ndeg", [(16, 14000), (0, 60000)])
 def test_mpnn_forward_tile_ranges(fe, ndeg):
     """The edge-parallel MPNN forward gives each wave one contiguous range of 32-edge tiles: a row split over
