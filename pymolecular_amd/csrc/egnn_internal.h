@@ -305,6 +305,12 @@ int mpnn_ep_blocks(int64_t E);
 // from L2, backward writes the per-edge weight-gradient factors Dm1, Dm, Dgq, Dga2.
 bool wide_supported(const LayerShape& s);
 int launch_wide_fwd(const LayerShape& s, const FwdArgs& a, hipStream_t st);
+// The edge-parallel forward (egnn_wfwd.hip) takes 25 us (MPNN 16) for any graph of less than a pass of its 2,048 waves,
+// one wave's latency; the kernel that shares a 32-edge tile over eight waves takes 13 us (9) for a pass of 256 tiles and 7 (5)
+// for each further one.  Measured, edge-parallel against shared: 1,000 edges 25.1 / 13.3 us (16.4 / 9.3), 8,192 25.4 / 14.4
+// (16.2 / 10.1), 16,384 26.0 / 21.8 (16.8 / 15.0), 20,000 25.8 / 28.4 (16.6 / 19.2), 50,000 37 / 55 (23 / 38).
+inline bool wide_fwd_ep(int64_t E) { return E > 2 * 256 * kTileEdges; }
+int launch_wide_fwd_ep(const LayerShape& s, const FwdArgs& a, hipStream_t st);
 // The backward runs one persistent 16-wave block per CU and writes per-block partials of dw2_mov
 // and dw_d ([nblk][M | H], EGNN) to BwdArgs::dwpart.
 constexpr int kWideBwdBlocks = 256;

@@ -88,6 +88,17 @@ __device__ __forceinline__ int rank_of(uint32_t mask, int k) {
   return __popc(mask & below) - 1;
 }
 
+// B operand S[edge][rank]: column n = rank 16*rb + c, rows = edges kappa_chain(g, s)
+__device__ __forceinline__ bf16x8 seg_chunk(uint32_t mask, int nvalid, int rb, int c, int g) {
+  bf16x8 r;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int k = kappa_chain(g, s);
+    r[s] = (k < nvalid && rank_of(mask, k) == 16 * rb + c) ? (bf16)1.0f : (bf16)0.0f;
+  }
+  return r;
+}
+
 // P_i + Q_j of a 16-feature block from one gathered B chunk: lanes g = 0, 1 of
 // edge column c hold P features 8g .. 8g + 7 of the block, lanes g = 2, 3 Q
 // features 8(g - 2) .. + 7 (pq_gather); A[r][k] = 1 where k is P or Q feature r.

@@ -31,8 +31,8 @@ def test_many_passes(E, eq):
 
 @pytest.mark.parametrize("eq,fe", [(True, 32), (True, 56), (False, 8)])
 def test_same_bits_on_both_sides_of_the_rule(eq, fe):
-    """A graph of 8,192 edges (the kernel that shares a tile) alone and as the first part of one of 17,600 (the
-    edge-parallel kernel): the gradient of its nodes' features is the same to the bit, as every stage of the two kernels
+    """A graph of 8,192 edges (the kernels that share a tile) alone and as the first part of one of 17,600 (the
+    edge-parallel kernels): its messages and the gradient of its nodes' features are the same to the bit, as every stage
     sums in the same order."""
     part, rest = [32] * 256, [40] * 235 + [8, 0]
     rowptr, col = random_csr(256, part, seed=9)

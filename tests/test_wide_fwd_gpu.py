@@ -1,4 +1,5 @@
-"""Edge-parallel forward at H = 256 (bf16) at the edges of its tiles and passes, against the oracle."""
+"""Forward at H = 256 (bf16) at the edges of tiles and passes, against the oracle: up to 16,384 edges the kernel that shares
+a tile over eight waves, beyond them the edge-parallel one."""
 import numpy as np
 import pytest
 
@@ -27,6 +28,17 @@ def test_edge_slots(eq, fe):
     check_case(Case(rowptr, col, 64, fe, 256, 256, 256, seed=52, eq=eq, edge_ids=perm), "bf16")
 
 
+@pytest.mark.parametrize("eq,fe", [(True, 0), (True, 32), (True, 56), (False, 8), (False, 64)])
+@pytest.mark.parametrize("kind", ["none", "one", "15", "17", "33", "ones", "halves", "long"])
+def test_edge_parallel_tiles(kind, eq, fe):
+    """The same tails behind 16,384 edges in rows of 32 (whole tiles, 512 of them: without a tail the tile-sharing kernel's
+    last graph), one and two 32-slot slices of edge inputs, permuted edge ids."""
+    degs = [32] * 512 + ([] if kind == "none" else _degrees(kind)) + [0] * 5
+    rowptr, col = random_csr(len(degs), degs, seed=len(degs))
+    perm = np.random.Generator(np.random.PCG64(4)).permutation(len(col))
+    check_case(Case(rowptr, col, 32, fe, 256, 256, 256, seed=55, eq=eq, mean_agg=eq, edge_ids=perm), "bf16", backward=False)
+
+
 def test_many_passes():
     """More tiles than one pass of the grid (512 blocks of four tiles)."""
     degs = np.full(2100, 33)
@@ -37,8 +49,9 @@ def test_many_passes():
 @pytest.mark.parametrize("eq", [True, False])
 def test_infinite_feature(eq):
     """One infinite entry of b1: an infinite message where its weight is positive, SiLU(-inf) = NaN where it is negative,
-    as in the oracle (rows of 32 edges, so that no row sum multiplies another row's infinity by 0)."""
-    rowptr, col = random_csr(40, np.full(40, 32), seed=8)
+    as in the oracle (the edge-parallel kernel; rows of 32 edges, so that no row sum multiplies another row's infinity
+    by 0)."""
+    rowptr, col = random_csr(520, np.full(520, 32), seed=8)
     case = Case(rowptr, col, 32, 8, 256, 256, 256, seed=54, eq=eq)
     case.p["b1"][37] = np.inf
     got = run_fused(case, "bf16", backward=False)["out_msg"]
