@@ -39,13 +39,20 @@ constexpr int kScanRows = 2048, kSortMax = 512;
 // list in registers: 334 k edges 36 us in four launches against 120 us in 24 with the library's sort.  The scatter's
 // cost grows with the spread of the sources, so the two cross between 0.9M and 2M edges by kind of graph; the line lies
 // below all of them.  One schedule, counting / sort: chains with kNN edges 983k 120 / 213 us, 1.97M 173 / 174, 3.9M
-// 278 / 257; random sources 1.28M 251 / 165, 2.56M 422 / 179; power law 0.87M 193 / 253, 1.40M 273 / 210, and with the
-// hubs as sources (lists past kSortMax: counted in vain, then sorted) 0.87M 290 / 243.
+// 278 / 257; random sources 1.28M 251 / 165, 2.56M 422 / 179; power law 0.87M 193 / 253, 1.40M 273 / 210.
 constexpr int64_t kCountMaxEdges = int64_t(3) << 18;
+
+// Atomics on one address follow each other, so a few hubs that hold most edges as sources would make the count the slowest
+// part (600k edges from 20 sources 1,646 us; the sort 221).  The launch that clears the counts looks at kHubSample edges
+// and leaves the graph to the sort when so many of them share a source (of a hash, so rarely two) that its list is likely
+// longer than kSortMax.  One schedule of 600k edges, before / with the check / by the sort alone: 20 hubs 1,646 / 214 /
+// 221 us, one hub with 1 % of the edges 284 / 218 / 225, none 133 / 138 / 226.
+constexpr int kHubSample = 4096, kHubHits = 6, kHubHash = 16384;
+constexpr int32_t kNotCounted = 0x7fffffff;   // in place of the longest list
 
 struct SchedTmp {
   int32_t* cnt;       // [N] edges per source, then each list's fill position
-  int32_t* state;     // [2] CSR error, longest source list (right after cnt: cleared together)
+  int32_t* state;     // [2] CSR error, longest source list
   int32_t* bsum;      // [scan blocks][2] per block: edges, fix rows
   int32_t* keys_out;
   int32_t* vals_in;
@@ -85,9 +92,37 @@ size_t schedule_tmp_bytes(int64_t N, int64_t E) {
   return tmp_layout(N, E, nullptr, &t);
 }
 
+// clears cnt and state; block 0 looks for hubs (hubs != 0): state[1] = kNotCounted
+__global__ __launch_bounds__(256) void clear_kernel(const int32_t* __restrict__ col, int64_t N, int64_t E,
+                                                    int32_t* __restrict__ cnt, int32_t* __restrict__ state, int hubs) {
+  __shared__ int32_t hits[kHubHash];
+  for (int64_t q = blockIdx.x * (int64_t)256 + threadIdx.x; q < N; q += (int64_t)gridDim.x * 256) cnt[q] = 0;
+  if (blockIdx.x > 0) return;
+  int found = 0;
+  if (hubs) {
+    int32_t j[kHubSample / 256];
+#pragma unroll
+    for (int k = 0; k < kHubSample / 256; ++k) j[k] = col[(threadIdx.x + 256 * k) * E / kHubSample];
+    for (int q = threadIdx.x; q < kHubHash; q += 256) hits[q] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kHubSample / 256; ++k) {
+      const int64_t n = atomicAdd(&hits[((uint32_t)j[k] * 2654435761u) >> 18], 1) + 1;
+      if (n >= kHubHits && n * E > (int64_t)kHubSample * kSortMax) found = 1;
+    }
+  }
+  found = __syncthreads_or(found);
+  if (threadIdx.x == 0) {
+    state[0] = 0;
+    state[1] = found ? kNotCounted : 0;
+  }
+}
+
 // CSR checks and (cnt != null) the number of edges per source
 __global__ void csr_count_kernel(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col, int64_t N,
-                                 int64_t E, int32_t* __restrict__ cnt, int32_t* err) {
+                                 int64_t E, int32_t* __restrict__ cnt, int32_t* state) {
+  int32_t* const err = state;
+  if (state[1] == kNotCounted) cnt = nullptr;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   int bad = 0;
@@ -349,9 +384,10 @@ int launch_schedule(const int32_t* rowptr, const int32_t* col, int64_t N, int64_
                     size_t tmp_bytes, hipStream_t st) {
   SchedTmp t;
   if (tmp_layout(N, E, tmp, &t) > tmp_bytes) return EGNN_ERR_WORKSPACE;
-  if (hipMemsetAsync(t.cnt, 0, sizeof(int32_t) * (size_t)(N + 2), st) != hipSuccess) return EGNN_ERR_HIP;
   int vb = (int)std::min<int64_t>(cdiv(std::max(N, E), 256), 4096);
-  const bool count = E <= kCountMaxEdges;   // else the fix rows alone come from the scan (of zero counts)
+  bool count = E <= kCountMaxEdges;   // else the fix rows alone come from the scan (of zero counts)
+  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)std::min<int64_t>(cdiv(N, 1024), 1024)), dim3(256), 0, st, col, N, E, t.cnt,
+                     t.state, count && E > kSortMax ? 1 : 0);
   hipLaunchKernelGGL(csr_count_kernel, dim3(vb), dim3(256), 0, st, rowptr, col, N, E, count ? t.cnt : nullptr, t.state);
   const int64_t sb = cdiv(N, kScanRows);
   hipLaunchKernelGGL(scan_sums_kernel, dim3((unsigned)sb), dim3(256), 0, st, rowptr, t.cnt, N, t.bsum, t.state + 1);
@@ -359,6 +395,7 @@ int launch_schedule(const int32_t* rowptr, const int32_t* col, int64_t N, int64_
   if (hipMemcpyAsync(host, t.state, sizeof(host), hipMemcpyDeviceToHost, st) != hipSuccess) return EGNN_ERR_HIP;
   if (hipStreamSynchronize(st) != hipSuccess) return EGNN_ERR_HIP;
   if (host[0]) return EGNN_ERR_CSR;
+  count = count && host[1] != kNotCounted;
 
   const bool mid = sb > 1024;
   if (mid) hipLaunchKernelGGL(scan_mid_kernel, dim3(1), dim3(256), 0, st, t.bsum, sb);

@@ -29,6 +29,17 @@ def test_source_list_lengths(lens):
     _check(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32), col)
 
 
+@pytest.mark.parametrize("E,hubs,share", [(512, 1, 1.0), (513, 1, 1.0), (40_000, 1, 0.5), (100_000, 5, 1.0), (100_000, 40, 1.0),
+                                          (300_000, 1, 0.01), (786_432, 20, 0.9)])
+def test_hub_sources(E, hubs, share):
+    """Few sources with most of the edges, around the sampled rule that leaves them to the radix sort."""
+    r = np.random.Generator(np.random.PCG64(E + hubs))
+    N = 5000
+    col = np.where(r.random(E) < share, r.integers(0, hubs, size=E) * 97, r.integers(0, N, size=E)).astype(np.int32)
+    deg = np.bincount(r.integers(0, N, size=E), minlength=N)
+    _check(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32), col)
+
+
 @pytest.mark.parametrize("N", [1, 2047, 2048, 2049, 65536, 65537, 2048 * 1025 + 3])
 def test_scan_block_edges(N):
     """Node counts around one block of the scan, the two row-id launches, and the separate prefix launch."""
