@@ -213,8 +213,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
             __builtin_amdgcn_sched_barrier(0);
             f32x4 lo3[2] = {zero4(), zero4()};
             mma3x2(q + rb, lo3, A.a, A.b, mc);
-            q[rb] = joined(q[rb], lo3[0]);
-            q[rb + 1] = joined(q[rb + 1], lo3[1]);
+            q[rb] += lo3[0];   // not joined: an infinite message makes phi NaN by its SiLU(-inf) too
+            q[rb + 1] += lo3[1];
             __builtin_amdgcn_sched_barrier(0);
             A = An;
           }
@@ -374,8 +374,9 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
     stream_store(ch + 1, 1);
     __syncthreads();
   };
-  // one k slice of the second: acc[rb] += A[rb] . B
-  auto slice_chunk = [&](int ch, const Chunk3& B, f32x4* acc) {
+  // one k slice of the second: acc[rb] += A[rb] . B; inf: infinities are kept (S5; in the recomputation an infinite
+  // activation ends in SiLU' = NaN in any case)
+  auto slice_chunk = [&](int ch, const Chunk3& B, f32x4* acc, auto inf) {
     const bf16* W = s_w[ch & 1];
     stream_load(ch + 1, 0);
     Chunk3 A = lds_chunk3(W, l);
@@ -386,7 +387,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       f32x4 lo = zero4();
       mma3(acc[rb], lo, A, B);
-      acc[rb] = joined(acc[rb], lo);
+      acc[rb] = inf ? joined(acc[rb], lo) : acc[rb] + lo;
       __builtin_amdgcn_sched_barrier(0);
       A = An;
       if (rb == 3) {
@@ -459,7 +460,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
             const Chunk3 A = lds_chunk3((const bf16*)a.fr.s_u + ((int64_t)(rb >> 1) * 6 * a.NUC + ((rb & 1) * a.NUC + uc) * 3) * kFragElems, l);
             f32x4 lo = zero4(), hi = zero4();
             mma3(hi, lo, A, u3);
-            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], joined(hi, lo), sg);
+            y[rb >> 1][rb & 1] = add_signed(y[rb >> 1][rb & 1], hi + lo, sg);
           }
         }
       } else if constexpr (EQ) {
@@ -501,16 +502,16 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
       f32x4 x[2];
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g), p2 = joined(hi[b], lo[b]);
+        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 32 * kp + 16 * b + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(__builtin_fmaf(p2[i], sg, b2[i]), sg);
+          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
           x[b][i] = r.y;
           s2[kp][b][i] = r.d;
         }
         if (EQ && valid) *reinterpret_cast<f32x4*>((float*)a.Dm + fo + 32 * kp + 16 * b) = x[b];
       }
-      if constexpr (EQ) slice_chunk(2 * kp + 1, split_chunk(x[0], x[1]), q);
+      if constexpr (EQ) slice_chunk(2 * kp + 1, split_chunk(x[0], x[1]), q, std::false_type());
     }
     // ---- phi, g_q, dw2_mov
     float phi = 0.f;
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
         x[b] *= s2[kp][b];
         if (valid) *reinterpret_cast<f32x4*>((float*)a.Dga2 + fo + 32 * kp + 16 * b) = x[b];
       }
-      slice_chunk(EQ ? 2 * KP + 2 * kp + 1 : KP + kp, split_chunk(x[0], x[1]), ga1);
+      slice_chunk(EQ ? 2 * KP + 2 * kp + 1 : KP + kp, split_chunk(x[0], x[1]), ga1, std::true_type());
     }
     // ---- Gh, S6, dw_d
     {

@@ -174,11 +174,9 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
         const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 16 * b + 4 * g);
         const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g);
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          const f32x4 p = joined(hi[nb], lo[nb]);
+        for (int nb = 0; nb < 2; ++nb)   // not joined: an infinite message makes phi NaN by its SiLU(-inf) too
 #pragma unroll
-          for (int i = 0; i < 4; ++i) phi[nb] += silu_f32(__builtin_fmaf(p[i], sg, bx[i])) * w2[i];
-        }
+          for (int i = 0; i < 4; ++i) phi[nb] += silu_f32(__builtin_fmaf(hi[nb][i] + lo[nb][i], sg, bx[i])) * w2[i];
       }
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
@@ -433,8 +431,8 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         for (int rb = 0; rb < 4; rb += 2) {
           f32x4 hi[2] = {zero4(), zero4()}, lo[2] = {zero4(), zero4()};
           mma3x2(hi, lo, frag3(s_u + rb * 3 * kFragElems, l), frag3(s_u + (rb + 1) * 3 * kFragElems, l), u3);
-          y[rb] = add_signed(y[rb], joined(hi[0], lo[0]), sg);
-          y[rb + 1] = add_signed(y[rb + 1], joined(hi[1], lo[1]), sg);
+          y[rb] = add_signed(y[rb], hi[0] + lo[0], sg);
+          y[rb + 1] = add_signed(y[rb + 1], hi[1] + lo[1], sg);
         }
         opaque(u.lo);   // split again for d[W_e | w_d]
         opaque(u.hi);
@@ -462,10 +460,10 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
         mma3x2(hi, lo, w_cols3<H>(s_hl, 0, kc, c, g), w_cols3<H>(s_hl, 1, kc, c, g), m1[kc]);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 16 * b + 4 * g), p = joined(hi[b], lo[b]);
+        const f32x4 b2 = *reinterpret_cast<const f32x4*>(s_vec + 16 * b + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(__builtin_fmaf(p[i], sg, b2[i]), sg);
+          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, b2[i]), sg);
           x[b][i] = r.y;
           s2[b][i] = r.d;
         }
@@ -483,10 +481,10 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         const f32x4 bx = *reinterpret_cast<const f32x4*>(s_vec + O + 16 * b + 4 * g);
-        const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g), p = joined(hi[b], lo[b]);
+        const f32x4 w2 = *reinterpret_cast<const f32x4*>(s_vec + O + M + 16 * b + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const YD r = silu_yd_f32(__builtin_fmaf(p[i], sg, bx[i]), sg);
+          const YD r = silu_yd_f32(__builtin_fmaf(hi[b][i] + lo[b][i], sg, bx[i]), sg);
           phi += r.y * w2[i];
           pb[b][i] = gphi * r.y;
           gv[b][i] = gphi * w2[i] * r.d;

@@ -47,7 +47,7 @@ constexpr int64_t kCountMaxEdges = int64_t(3) << 18;
 // and leaves the graph to the sort when so many of them share a source (of a hash, so rarely two) that its list is likely
 // longer than kSortMax.  One schedule of 600k edges, before / with the check / by the sort alone: 20 hubs 1,646 / 214 /
 // 221 us, one hub with 1 % of the edges 284 / 218 / 225, none 133 / 138 / 226.
-constexpr int kHubSample = 4096, kHubHits = 6, kHubHash = 16384;
+constexpr int kHubSample = 4096, kHubHits = 6, kHubHash = 16384, kClear = 1024;   // threads of the launch
 constexpr int32_t kNotCounted = 0x7fffffff;   // in place of the longest list
 
 struct SchedTmp {
@@ -93,20 +93,20 @@ size_t schedule_tmp_bytes(int64_t N, int64_t E) {
 }
 
 // clears cnt and state; block 0 looks for hubs (hubs != 0): state[1] = kNotCounted
-__global__ __launch_bounds__(256) void clear_kernel(const int32_t* __restrict__ col, int64_t N, int64_t E,
+__global__ __launch_bounds__(kClear) void clear_kernel(const int32_t* __restrict__ col, int64_t N, int64_t E,
                                                     int32_t* __restrict__ cnt, int32_t* __restrict__ state, int hubs) {
   __shared__ int32_t hits[kHubHash];
-  for (int64_t q = blockIdx.x * (int64_t)256 + threadIdx.x; q < N; q += (int64_t)gridDim.x * 256) cnt[q] = 0;
+  for (int64_t q = blockIdx.x * (int64_t)kClear + threadIdx.x; q < N; q += (int64_t)gridDim.x * kClear) cnt[q] = 0;
   if (blockIdx.x > 0) return;
   int found = 0;
   if (hubs) {
-    int32_t j[kHubSample / 256];
+    int32_t j[kHubSample / kClear];
 #pragma unroll
-    for (int k = 0; k < kHubSample / 256; ++k) j[k] = col[(threadIdx.x + 256 * k) * E / kHubSample];
-    for (int q = threadIdx.x; q < kHubHash; q += 256) hits[q] = 0;
+    for (int k = 0; k < kHubSample / kClear; ++k) j[k] = col[(threadIdx.x + kClear * k) * E / kHubSample];
+    for (int q = threadIdx.x; q < kHubHash; q += kClear) hits[q] = 0;
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kHubSample / 256; ++k) {
+    for (int k = 0; k < kHubSample / kClear; ++k) {
       const int64_t n = atomicAdd(&hits[((uint32_t)j[k] * 2654435761u) >> 18], 1) + 1;
       if (n >= kHubHits && n * E > (int64_t)kHubSample * kSortMax) found = 1;
     }
@@ -386,7 +386,7 @@ int launch_schedule(const int32_t* rowptr, const int32_t* col, int64_t N, int64_
   if (tmp_layout(N, E, tmp, &t) > tmp_bytes) return EGNN_ERR_WORKSPACE;
   int vb = (int)std::min<int64_t>(cdiv(std::max(N, E), 256), 4096);
   bool count = E <= kCountMaxEdges;   // else the fix rows alone come from the scan (of zero counts)
-  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)std::min<int64_t>(cdiv(N, 1024), 1024)), dim3(256), 0, st, col, N, E, t.cnt,
+  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)std::min<int64_t>(cdiv(N, 2 * kClear), 512)), dim3(kClear), 0, st, col, N, E, t.cnt,
                      t.state, count && E > kSortMax ? 1 : 0);
   hipLaunchKernelGGL(csr_count_kernel, dim3(vb), dim3(256), 0, st, rowptr, col, N, E, count ? t.cnt : nullptr, t.state);
   const int64_t sb = cdiv(N, kScanRows);
