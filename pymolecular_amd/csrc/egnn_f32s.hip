@@ -65,7 +65,7 @@ __global__ __launch_bounds__(64 * kW, 3) void f32s_fwd_kernel(FwdArgs a) {
   __shared__ __attribute__((aligned(16))) float s_msg[kW][kTileEdges * SP];
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, g = l >> 4;
-  const float sg = c & 1 ? -1.0f : 1.0f;   // the edge's sign in the chain
+  const float sg = bitsf(0x3f800000u | (uint32_t)(c & 1) << 31);   // the edge's sign in the chain, 1 or -1
   const float* PQ = (const float*)a.PQ;
   const float* ef = (const float*)a.ef;
   const int64_t E = a.E;
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(64 * kW, 2) void f32s_bwd_kernel(BwdArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 s_x[kW][4 * kSlot];
 
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l & 15, g = l >> 4;
-  const float sg = c & 1 ? -1.0f : 1.0f;   // the edge's sign in the chain
+  const float sg = bitsf(0x3f800000u | (uint32_t)(c & 1) << 31);   // the edge's sign in the chain, 1 or -1
   const float* PQ = (const float*)a.PQ;
   const float* ef = (const float*)a.ef;
   const float* gmsg = (const float*)a.gmsg;

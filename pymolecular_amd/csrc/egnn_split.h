@@ -116,7 +116,7 @@ __device__ __forceinline__ float sigmoid_f32(float x, float sg = 1.0f) {
   const float t = u * -1.44269502e+0f;                                   // fl(log2 e)
   const float d = __builtin_fmaf(u, -1.92596303e-8f, __builtin_fmaf(u, -1.44269502e+0f, -t));
   const float e = __builtin_amdgcn_exp2f(t);
-  return __builtin_amdgcn_rcpf(__builtin_fmaf(e * __builtin_fmaf(d, 0.693147182f, 1.0f), sg, sg));   // e may be inf: a product first
+  return __builtin_amdgcn_rcpf(__builtin_fmaf(e, __builtin_fmaf(d, 0.693147182f * sg, sg), sg));   // e may be inf: rcp 0
 }
 __device__ __forceinline__ float silu_f32(float x, float sg = 1.0f) { return x * sigmoid_f32(x, sg); }
 __device__ __forceinline__ YD silu_yd_f32(float x, float sg = 1.0f) {
