@@ -43,11 +43,14 @@ constexpr int kScanRows = 2048, kSortMax = 512;
 constexpr int64_t kCountMaxEdges = int64_t(3) << 18;
 
 // Atomics on one address follow each other, so a few hubs that hold most edges as sources would make the count the slowest
-// part (600k edges from 20 sources 1,646 us; the sort 221).  The launch that clears the counts looks at kHubSample edges
-// and leaves the graph to the sort when so many of them share a source (of a hash, so rarely two) that its list is likely
-// longer than kSortMax.  One schedule of 600k edges, before / with the check / by the sort alone: 20 hubs 1,646 / 214 /
-// 221 us, one hub with 1 % of the edges 284 / 218 / 225, none 133 / 138 / 226.
-constexpr int kHubSample = 4096, kHubHits = 6, kHubHash = 16384, kClear = 1024;   // threads of the launch
+// part.  The launch that clears the counts looks at kHubSample edges, a run of kHubRun (one cache line) at a scattered place
+// in each of kClear equal pieces, so that no row length fits the distance, and leaves the graph to the sort when so many of
+// them share a source (of a hash, so rarely two) that its list is likely longer than kSortMax.  One schedule of 600k edges,
+// without / with the check: 5 hubs 3,033 / 212 us, 20 hubs 1,631 / 216, one hub with 1 % of the edges 282 / 221; flat lists
+// of 123k, 614k and 640k edges 71 / 70, 101 / 99 and 153 / 153.  (Single edges instead of runs, 4,096 lines read by one
+// block, added 5 us to each.)
+constexpr int kClear = 1024;   // threads of the launch
+constexpr int kHubRun = 4, kHubSample = kClear * kHubRun, kHubHits = 6, kHubHash = 16384;
 constexpr int32_t kNotCounted = 0x7fffffff;   // in place of the longest list
 
 struct SchedTmp {
@@ -100,13 +103,16 @@ __global__ __launch_bounds__(kClear) void clear_kernel(const int32_t* __restrict
   if (blockIdx.x > 0) return;
   int found = 0;
   if (hubs) {
-    int32_t j[kHubSample / kClear];
+    const int64_t lo = threadIdx.x * E / kClear, len = (threadIdx.x + 1) * E / kClear - lo;
+    const int64_t at = lo + ((int64_t)((threadIdx.x * 2654435761u) >> 8) * len >> 24);
+    const int32_t* p = col + min(at, E - kHubRun);   // E > kSortMax
+    int32_t j[kHubRun];
 #pragma unroll
-    for (int k = 0; k < kHubSample / kClear; ++k) j[k] = col[(threadIdx.x + kClear * k) * E / kHubSample];
+    for (int k = 0; k < kHubRun; ++k) j[k] = p[k];
     for (int q = threadIdx.x; q < kHubHash; q += kClear) hits[q] = 0;
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kHubSample / kClear; ++k) {
+    for (int k = 0; k < kHubRun; ++k) {
       const int64_t n = atomicAdd(&hits[((uint32_t)j[k] * 2654435761u) >> 18], 1) + 1;
       if (n >= kHubHits && n * E > (int64_t)kHubSample * kSortMax) found = 1;
     }
