@@ -14,7 +14,7 @@
 // Row sums: each wave adds up its half's rows from its own LDS rows, one feature per lane, in edge order;
 // the first wave of a tile hands the sum of a row that goes on into the second half over through LDS.
 // Measured against one wave per 32-edge tile on the fp32 instruction with the weights read from L2 (E = 394k,
-// 46k and 0.7k edges of 9..29-atom molecules): 564 -> 233, 99 -> 34 and 51 -> 16 us.  What bounds it now is the
+// 46k and 0.7k edges of 9..29-atom molecules): 564 -> 236, 99 -> 36 and 51 -> 16 us.  What bounds it now is the
 // issue of the 768 products and about 2,400 vector instructions per wave and pass.
 #include "egnn_device.h"
 #include "egnn_internal.h"
@@ -311,7 +311,8 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_fwd_kernel(FwdArgs a) {
 // for atb_f32_kernel, all four with the edge's sign (odd edges negative: the products are the same); dw2_mov = sum g_phi p and dw_d = sum r^2 g_a1 are summed here (edge_sum16 over the wave's
 // edges, then registers over the passes) into one partial row [M | H] per block.
 // Measured against one wave per 32-edge tile on the fp32 instruction, which also stored p and r^2 for dw2_mov and
-// dw_d: 989 -> 527 us at 394k edges, 146 -> 90 us at 46k (both in two chunks).
+// dw_d: 989 -> 502 us at 384k edges (both in two chunks), 146 (two) -> 67 us (one) at 46k.  30 registers spill (38 with
+// edge features): vector 0.35 and matrix issue 0.25 of the cycles, 0.48 of the wave cycles waiting.
 template <bool EQ, bool FEAT>
 __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
   constexpr int H = 128, O = 128, M = 128, KH = H / 32, KP = O / 32, NCH = EQ ? 4 * KP : 2 * KP;
@@ -622,7 +623,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void f32_bwd_kernel(BwdArgs a) {
 // without bank conflicts), two slices in flight in registers and two in LDS.  The ones row (bias gradient) is the
 // sum of the B values each thread loads, in fp32, odd edges subtracted (their rows are stored negative).  Each block adds to its partial row of an earlier chunk.
 // Measured (both products, two chunks, with the matrix-vector products the backward kernel now sums itself):
-// 750 -> 222 us at 394k edges (3.6 TB/s), 123 -> 41 us at 46k.
+// 750 -> 222 us at 394k edges (3.6 TB/s), 123 -> 27 us at 46k (one chunk).
 constexpr int kAtbPitch = 144, kAtbSlice = 32, kAtbThreads = 512;
 constexpr int kAtbPlane = kAtbSlice * kAtbPitch;
 __device__ __forceinline__ bf16x8 tr_chunk(const bf16* p) {   // rows p + 0..3 and + 16..19 of the lane's k group

@@ -7,7 +7,7 @@
 // next stage's B operand.  Two blocks of four waves (forward: three) per CU; vector instructions (SiLU, the splits)
 // bound both kernels.
 // Measured against one wave per 32-edge tile on the fp32 instruction with the factors of the weight gradients in
-// memory (E = 1.28M, F_E = 16): forward 306 -> 166 us; backward and its weight gradients 1,990 -> 432 us, 52 -> 2
+// memory (E = 1.28M, F_E = 16): forward 306 -> 168 us; backward and its weight gradients 1,990 -> 444 us, 52 -> 2
 // launches.
 #include "egnn_device.h"
 #include "egnn_internal.h"

@@ -10,10 +10,10 @@
 // products of the current one and stored after them, one barrier per chunk, 16 chunks for 128 edges.  dw2_mov = sum g_phi p and
 // dw_d = sum r^2 g_a1 are summed over the 16 edges by a halving exchange (16 values a lane -> one) and kept in
 // registers over the passes: one partial row [M | H] per block.
-// One block per CU, two waves per SIMD; vector and matrix issue (about 40 % of the cycles) and the waits of LDS operand
+// One block per CU, two waves per SIMD; vector and matrix issue (0.40 and 0.20 of the cycles) and the waits of LDS operand
 // reads and barriers bound it.
 // Measured against the kernel that shares a 32-edge tile over eight waves by feature rows (661k edges, F_E = 32):
-// 990 -> 815 us; the weights' loads through generic pointers, whose waits join those of the LDS, cost 20 us of it.
+// 990 -> 775 us; the weights' loads through generic pointers, whose waits join those of the LDS, cost 20 us of it.
 // Every stage sums in the order of egnn_wide.hip (biases, P_i and Q_j onto the finished products, g_m as the first term), so
 // the factors and Gh are bit for bit those of that kernel.
 // A lane past the last edge computes that edge again and stores the same values, so no store is under a branch.

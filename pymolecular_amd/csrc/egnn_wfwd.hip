@@ -15,7 +15,7 @@
 // transposing reads and multiplied by the 0/1 segment matrix of the schedule's rank table; whole rows are stored, the
 // tile's partial rows go to its carry slots, as do the coordinate sums (delta phi as a bf16 hi + lo pair).
 // Measured against the kernel whose eight waves share each tile by feature rows and exchange every stage through LDS
-// (660k and 44k edges, F_E = 32): 564 -> 341 and 49 -> 38 us.
+// (660k and 44k edges, F_E = 32): 564 -> 319 and 49 -> 38 us.
 #include "egnn_device.h"
 #include "egnn_internal.h"
 #include "egnn_tile.h"
