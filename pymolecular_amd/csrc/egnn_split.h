@@ -13,7 +13,7 @@
 // An infinite operand has no such parts: its second is inf - inf = NaN, which enters the correction terms only.  The two
 // accumulators are therefore added by joined(), which takes the large term alone where the corrections are NaN, so an
 // infinity comes out where the fp32 instruction gives one.  (Not in the weight gradients of egnn_f32s.hip, which keep both
-// in one accumulator, and not where NaN follows from SiLU(-inf) or SiLU'(inf) in any case.) 
+// in one accumulator, and not where NaN follows from SiLU(-inf) or SiLU'(inf) in any case.)
 // A finite operand never becomes infinite, as x0 is truncated; a NaN whose payload has its lower 16 bits only (no arithmetic
 // makes one) counts as an infinity.
 #pragma once
